@@ -459,6 +459,12 @@ __device__ __forceinline__ void gemm2(int m, int n, int k, const T *A0, const T 
     gemm_valu<TA, TB, T>(m, n, k, A0, A1, lda, B0, B1, ldb, C, ldc, false, 2, nb, sA, sB, sC);
 }
 
+template <typename T>
+__device__ __forceinline__ void set_one(T *p) {
+    if (threadIdx.x == 0) p[0] = (T)1;
+    __syncthreads();
+}
+
 // ---------------------------------------------------------------------------
 // GEMM: C(m x n) (+)= op(A) op(B).  op(A) is m x k: A(r,q) = TA ? A[q + lda*r] : A[r + lda*q].
 // FP32 products of useful size run on the matrix cores with the output tile

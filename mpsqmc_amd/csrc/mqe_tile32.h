@@ -17,6 +17,8 @@
 #ifndef MQE_TILE32_H
 #define MQE_TILE32_H
 
+#include "mqe_kernels.h"
+
 namespace mqe {
 namespace t32 {
 
@@ -42,7 +44,6 @@ enum : int {
     B_V = 12,    // 4 blocks
     NBLK = 16
 };
-constexpr int MAXG_T32 = 256;                    // grid points: four per lane of one wave
 
 constexpr size_t lds_bytes() { return sizeof(float) * (size_t)NBLK * BLK; }
 

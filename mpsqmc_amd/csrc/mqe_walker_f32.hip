@@ -1,0 +1,17 @@
+// mqe_walker_f32.hip -- the general walker kernel, FP32, bonds above 64.
+#include <hip/hip_runtime.h>
+
+#include "mqe_general.h"
+
+namespace mqe {
+
+void launch_walker_f32(const WalkerLaunch &l, const Sys &S, const Pool &P, const float *trial, int flags) {
+    hipLaunchKernelGGL((walker_kernel<float, false>), dim3(l.grid), dim3(MQE_NT), l.lds, l.stream, S, P, trial, flags);
+}
+
+hipError_t lds_attr_f32(size_t lds) {
+    return hipFuncSetAttribute((const void *)walker_kernel<float, false>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds);
+}
+
+}  // namespace mqe
