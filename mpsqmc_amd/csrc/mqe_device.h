@@ -883,6 +883,125 @@ __device__ __forceinline__ void householder_qr(const QRCols &col, int n, double 
     __syncthreads();
 }
 
+// sum over aligned groups of G = 4, 8 or 16 lanes; every lane receives it
+template <int G>
+__device__ __forceinline__ double lanes_sum(double v) {
+    v += dpp_d<0xB1>(v);                            // quad_perm [1,0,3,2]
+    v += dpp_d<0x4E>(v);                            // quad_perm [2,3,0,1]
+    if constexpr (G >= 8) v += dpp_d<0x141>(v);   // row_half_mirror
+    if constexpr (G >= 16) v += dpp_d<0x140>(v);  // row_mirror
+    return v;
+}
+
+// ---------------------------------------------------------------------------
+// The same factorisation with every column in registers: LPC lanes own a column
+// (lane ln its rows ln + LPC t, t < NE), so m <= LPC NE and n <= 256 / LPC; only
+// the reflectors (V, ld m, in LDS) and tau pass through LDS.  The group of column
+// j + 1 forms its reflector as soon as it has applied reflector j: one barrier
+// per column.  load(r, c): element of A (called once per element, before the
+// first barrier); put_r(r, c, x): R(r, c) for r <= c, after the last barrier
+// (V may be overwritten there if want_q is false); want_q: put_q(r, c, x) gets
+// Q, after a barrier past the last read of V.  Ends without a barrier.
+// What bounds it: the chain of one column (LDS read, dot product, group sum,
+// norm, root and division, LDS write, barrier), which nothing overlaps within a
+// walker; columns in LDS or memory put two to three more loads on that chain.
+// ---------------------------------------------------------------------------
+template <int LPC, int NE, class Load, class PutR, class PutQ>
+__device__ __forceinline__ void qr_regs(int m, int n, double *V, double *tau, bool want_q, Load load, PutR put_r,
+                                        PutQ put_q) {
+    const int g = threadIdx.x / LPC, ln = threadIdx.x % LPC;
+    double a[NE];
+#pragma unroll
+    for (int t = 0; t < NE; ++t) {
+        const int r = ln + LPC * t;
+        a[t] = r < m && g < n ? load(r, g) : 0.0;
+    }
+    __syncthreads();  // V may overlay what load() reads
+    auto reflect = [&](int j) {
+        double ss = 0.0, alpha = 0.0;
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            const int r = ln + LPC * t;
+            if (r > j) ss += a[t] * a[t];
+            if (r == j) alpha = a[t];
+        }
+        ss = lanes_sum<LPC>(ss);
+        alpha = lanes_sum<LPC>(alpha);
+        double tj = 0.0, sc = 0.0, beta = alpha;
+        if (ss != 0.0) {
+            beta = -copysign(sqrt(alpha * alpha + ss), alpha);
+            tj = (beta - alpha) / beta;
+            sc = 1.0 / (alpha - beta);
+        }
+        double *vj = V + (size_t)m * j;
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            const int r = ln + LPC * t;
+            if (r > j && r < m) {
+                a[t] *= sc;
+                vj[r] = a[t];
+            }
+            if (r == j) a[t] = beta;
+        }
+        if (ln == 0) tau[j] = tj;
+    };
+    // x <- H_j x, x in the rows of this lane
+    auto apply = [&](int j, double tj, double (&x)[NE]) {
+        const double *vj = V + (size_t)m * j;
+        double vr[NE], s = 0.0;
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            const int r = ln + LPC * t;
+            vr[t] = r > j && r < m ? vj[r] : (r == j ? 1.0 : 0.0);
+        }
+#pragma unroll
+        for (int t = 0; t < NE; ++t) s += vr[t] * x[t];
+        s = tj * lanes_sum<LPC>(s);
+#pragma unroll
+        for (int t = 0; t < NE; ++t) x[t] -= s * vr[t];
+    };
+    if (g == 0) reflect(0);
+    __syncthreads();
+    for (int j = 0; j < n; ++j) {
+        if (g > j && g < n) {
+            apply(j, tau[j], a);
+            if (g == j + 1) reflect(j + 1);
+        }
+        __syncthreads();
+    }
+    if (g < n) {
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            const int r = ln + LPC * t;
+            if (r <= g) put_r(r, g, a[t]);
+        }
+    }
+    if (!want_q) return;
+    // Q column c = H_0 H_1 ... H_c e_c; the groups of a wave take the same
+    // reflector at the same time, so its LDS reads are broadcasts
+#pragma unroll
+    for (int t = 0; t < NE; ++t) a[t] = ln + LPC * t == g ? 1.0 : 0.0;
+    for (int k = min(n - 1, (int)((threadIdx.x | 63) / LPC)); k >= 0; --k)
+        if (k <= g) apply(k, tau[k], a);
+    __syncthreads();
+    if (g < n) {
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            const int r = ln + LPC * t;
+            if (r < m) put_q(r, g, a[t]);
+        }
+    }
+}
+
+// qr_regs with the split by size: 8 lanes a column up to 64 x 32, 4 lanes up to 128 x 64
+constexpr int QR_REGS_M = 128, QR_REGS_N = 64;
+template <class Load, class PutR, class PutQ>
+__device__ __forceinline__ void qr_in_regs(int m, int n, double *V, double *tau, bool want_q, Load load, PutR put_r,
+                                           PutQ put_q) {
+    if (m <= 64 && n <= 32) qr_regs<8, 8>(m, n, V, tau, want_q, load, put_r, put_q);
+    else qr_regs<4, 32>(m, n, V, tau, want_q, load, put_r, put_q);
+}
+
 // ---------------------------------------------------------------------------
 // Philox4x32-10 (Salmon, Moraes, Dror, Shaw, SC'11) counter-based RNG.
 // ---------------------------------------------------------------------------

@@ -103,65 +103,171 @@ __device__ __forceinline__ T *wel(const Pool &P, T *phi, int k, int dl, int dr, 
     return P.padded ? phi + (size_t)(2 * k + s) * 1024 + r + 32 * c : phi + P.woff[k] + r + (size_t)dl * (c + (size_t)dr * s);
 }
 
-template <typename T>
-__device__ void compress_bond(const Pool &P, T *phi, int *wv, int k, int D, bool movingright, double *X, double *V,
-                              double *sig, int *ord, int *sh_flag) {
+// One bond of a sweep.  theta = A_k A_{k+1} (2 dl x 2 dr) has rank at most the
+// bond dimension dm between them, so its singular values come from a matrix of
+// at most dm columns.  With F the site whose new tensor is orthonormal (moving
+// right A_k as 2 dl x dm, moving left A_{k+1}^T as 2 dr x dm) and G the other one
+// (dm x n), theta = F G (or its transpose):
+//   G^T = Q R (R only),  C = F R^T  (C = F G when n < dm),
+//   rows(C) < columns(C): C^T = Q' R', C <- R'^T,
+//   U, sigma of C;  F's site <- U, G's site <- (U^T F) G.
+// A bond that is not truncated (columns of C <= D, and every singular value
+// well above the cut) needs only an orthonormal basis of the range of C: U is
+// the Q of C = Q R, and no SVD is taken (the state and the bond dimension are
+// the same; the basis of the bond is another).  That is every bond of the second
+// sweep.  The others take one-sided Jacobi sweeps on the columns of C.
+// X ((2 Dmax + 1) x Dmax doubles): C, then G's new tensor; Y (the same size): R,
+// then U^T F.  Both in LDS for Dmax <= 64 (SM), else in global scratch.
+// What bounds it: the sequential column steps and Jacobi rounds of one walker
+// (128 walkers of the 16-site snake at D = 32: 58.7 ms with Jacobi on all
+// min(2 dl, 2 dr) columns in global memory, 3.06 ms now).
+template <typename T, bool SM>
+__device__ __forceinline__ void compress_bond(const Pool &P, T *phi, int *wv, int k, int D, bool movingright, double *X,
+                                              double *Y, double *sig, int *ord, int *sh_flag, double *red) {
     const int dl = wv[k], dm = wv[k + 1], dr = wv[k + 2];
-    const int m = 2 * dl, n = 2 * dr;
-    const bool tr = n > m;  // Jacobi on the columns of the orientation with fewer of them
-    const int rows = tr ? n : m, cols = tr ? m : n;
-    // Compose: theta(alpha + dl il, beta + dr ir) = sum_mid A_k[il](alpha, mid) A_{k+1}[ir](mid, beta)
-    for (int e = threadIdx.x; e < m * n; e += MQE_NT) {
-        const int row = e % m, col = e / m;
-        const int al = row % dl, il = row / dl, be = col % dr, ir = col / dr;
-        double s = 0.0;
-        for (int q = 0; q < dm; ++q)
-            s += (double)*wel(P, phi, k, dl, dm, il, al, q) * (double)*wel(P, phi, k + 1, dm, dr, ir, q, be);
-        if (tr) X[col + (size_t)rows * row] = s;
-        else X[row + (size_t)rows * col] = s;
-    }
-    __syncthreads();
-    jacobi_svd_columns(X, rows, cols, V, sig, sh_flag);
-    sort_descending(sig, cols, ord);
-    int keep = 0;
-    for (int j = 0; j < cols; ++j) keep += sig[ord[j]] >= SCHMIDT_CUT ? 1 : 0;
-    keep = max(1, min(keep, D));
-    // left singular vector j (length m) and right one (length n) of theta
-    auto u = [&](int j, int row) {
-        const int c = ord[j];
-        return tr ? V[row + (size_t)cols * c] : (sig[c] > 0.0 ? X[row + (size_t)rows * c] / sig[c] : 0.0);
+    const int m = movingright ? 2 * dl : 2 * dr, n = movingright ? 2 * dr : 2 * dl;
+    const int df = movingright ? dl : dr, dg = movingright ? dr : dl;  // outer bonds of F and G
+    const int kf = movingright ? k : k + 1, kg = movingright ? k + 1 : k;
+    // element of the site ks: outer index o of physical index s, inner index q; di: inner bond dimension
+    auto at = [&](int ks, int dout, int di, int s, int o, int q) -> T * {
+        return ks == k ? wel(P, phi, k, dout, di, s, o, q) : wel(P, phi, k + 1, di, dout, s, q, o);
     };
-    auto vt = [&](int j, int col) {
-        const int c = ord[j];
-        return tr ? (sig[c] > 0.0 ? X[col + (size_t)rows * c] / sig[c] : 0.0) : V[col + (size_t)cols * c];
+    auto F = [&](int row, int q) { return (double)*at(kf, df, dm, row >= df ? 1 : 0, row >= df ? row - df : row, q); };
+    auto G = [&](int q, int col) { return (double)*at(kg, dg, dm, col >= dg ? 1 : 0, col >= dg ? col - dg : col, q); };
+    const int tid = threadIdx.x, ldx = m + 1;
+    const int rc = n < dm ? n : dm;  // columns of C
+    auto nothing = [](int, int, double) {};
+    // R of the QR of a rows x cols matrix (rows >= cols) given by load, to Y (ld cols)
+    auto r_factor = [&](int rows, int cols, auto load) {
+        if constexpr (SM) {
+            qr_in_regs(rows, cols, Y, sig, false, load, [&](int i, int j, double x) { Y[i + (size_t)cols * j] = x; },
+                       nothing);
+            __syncthreads();
+        } else {  // in X's place (the caller fills X afterwards), R to Y
+            for (int e = tid; e < rows * cols; e += MQE_NT) X[e] = load(e % rows, e / rows);
+            __syncthreads();
+            householder_r(X, rows, cols, rows, sig);
+            for (int e = tid; e < cols * cols; e += MQE_NT)
+                if (e % cols <= e / cols) Y[e] = X[e % cols + (size_t)rows * (e / cols)];
+            __syncthreads();
+        }
     };
-    // Decompose: the new bond holds `keep` states (zero padding cleared on the tile layout)
-    if (P.padded) {
-        for (int e = threadIdx.x; e < 2 * 1024; e += MQE_NT) {
-            phi[(size_t)(2 * k) * 1024 + e] = (T)0;
-            phi[(size_t)(2 * k + 2) * 1024 + e] = (T)0;
+    auto build_C = [&]() {  // C to X
+        if (n >= dm) {
+            r_factor(n, dm, [&](int col, int q) { return G(q, col); });
+            // C = F R^T: C(i, j) = sum_{q >= j} F(i, q) R(j, q)
+            for (int e = tid; e < m * dm; e += MQE_NT) {
+                const int i = e % m, j = e / m;
+                double s = 0.0;
+#pragma unroll 8
+                for (int q = j; q < dm; ++q) s += F(i, q) * Y[j + (size_t)dm * q];
+                X[i + (size_t)ldx * j] = s;
+            }
+        } else {
+            for (int e = tid; e < m * n; e += MQE_NT) {
+                const int i = e % m, j = e / m;
+                double s = 0.0;
+#pragma unroll 8
+                for (int q = 0; q < dm; ++q) s += F(i, q) * G(q, j);
+                X[i + (size_t)ldx * j] = s;
+            }
         }
         __syncthreads();
+    };
+    build_C();
+    int r = rc, keep = 0;
+    bool basis_only = false;
+    if constexpr (SM) {
+        if (rc <= m && rc <= D) {
+            qr_in_regs(m, rc, X, sig, true, [&](int i, int j) { return X[i + (size_t)ldx * j]; },
+                       [&](int i, int j, double x) { Y[i + (size_t)rc * j] = x; },
+                       [&](int i, int j, double x) { X[i + (size_t)ldx * j] = x; });
+            __syncthreads();
+            // ten times the cut: the bound's own rounding cannot matter
+            basis_only = least_singular_bound(Y, rc, Y + (size_t)rc * rc, red) > 10 * SCHMIDT_CUT;
+            if (!basis_only) build_C();
+        }
     }
-    for (int e = threadIdx.x; e < m * keep; e += MQE_NT) {
-        const int row = e % m, j = e / m, al = row % dl, il = row / dl;
-        const double f = movingright ? 1.0 : sig[ord[j]];
-        *wel(P, phi, k, dl, keep, il, al, j) = (T)(u(j, row) * f);
+    if (basis_only) {
+        keep = rc;
+        for (int j = tid; j < rc; j += MQE_NT) {
+            sig[j] = 1.0;
+            ord[j] = j;
+        }
+        __syncthreads();
+    } else {
+        if (r > m) {
+            if constexpr (SM) {
+                r_factor(r, m, [&](int j, int i) { return X[i + (size_t)ldx * j]; });
+            } else {
+                for (int e = tid; e < m * r; e += MQE_NT) Y[e / m + (size_t)r * (e % m)] = X[e % m + (size_t)ldx * (e / m)];
+                __syncthreads();
+                householder_r(Y, r, m, r, sig);
+            }
+            const int ldy = SM ? m : r;
+            for (int e = tid; e < m * m; e += MQE_NT) {
+                const int i = e % m, j = e / m;
+                X[i + (size_t)ldx * j] = j <= i ? Y[j + (size_t)ldy * i] : 0.0;
+            }
+            r = m;
+            __syncthreads();
+        }
+        jacobi_left_vectors(X, m, r, ldx, sig, sh_flag);
+        sort_descending(sig, r, ord);
+        for (int j = 0; j < r; ++j) keep += sig[ord[j]] >= SCHMIDT_CUT ? 1 : 0;
+        keep = max(1, min(keep, D));
     }
-    for (int e = threadIdx.x; e < keep * n; e += MQE_NT) {
-        const int j = e % keep, col = e / keep, be = col % dr, ir = col / dr;
-        const double f = movingright ? sig[ord[j]] : 1.0;
-        *wel(P, phi, k + 1, keep, dr, ir, j, be) = (T)(vt(j, col) * f);
+    // U^T F (keep x dm) while F's site still holds F
+    for (int e = tid; e < keep * dm; e += MQE_NT) {
+        const int j = e % keep, q = e / keep, c = ord[j];
+        const double *u = X + (size_t)ldx * c;
+        double s = 0.0;
+#pragma unroll 8
+        for (int i = 0; i < m; ++i) s += u[i] * F(i, q);
+        Y[j + (size_t)keep * q] = sig[c] > 0.0 ? s / sig[c] : 0.0;
     }
     __syncthreads();
-    if (threadIdx.x == 0) wv[k + 1] = keep;
+    // the new bond holds `keep` states (zero padding cleared on the tile layout)
+    if (P.padded) {
+        for (int e = tid; e < 2 * 1024; e += MQE_NT) phi[(size_t)(2 * kf) * 1024 + e] = (T)0;
+        __syncthreads();
+    }
+    for (int e = tid; e < m * keep; e += MQE_NT) {
+        const int row = e % m, j = e / m, c = ord[j];
+        const double v = sig[c] > 0.0 ? X[row + (size_t)ldx * c] / sig[c] : 0.0;
+        *at(kf, df, keep, row >= df ? 1 : 0, row >= df ? row - df : row, j) = (T)v;
+    }
+    __syncthreads();
+    for (int e = tid; e < keep * n; e += MQE_NT) {
+        const int j = e % keep, col = e / keep;
+        double s = 0.0;
+#pragma unroll 8
+        for (int q = 0; q < dm; ++q) s += Y[j + (size_t)keep * q] * G(q, col);
+        X[e] = s;
+    }
+    __syncthreads();
+    if (P.padded) {
+        for (int e = tid; e < 2 * 1024; e += MQE_NT) phi[(size_t)(2 * kg) * 1024 + e] = (T)0;
+        __syncthreads();
+    }
+    for (int e = tid; e < keep * n; e += MQE_NT) {
+        const int j = e % keep, col = e / keep;
+        *at(kg, dg, keep, col >= dg ? 1 : 0, col >= dg ? col - dg : col, j) = (T)X[e];
+    }
+    if (tid == 0) wv[k + 1] = keep;
     __syncthreads();
 }
+
+// Doubles of one of the two work matrices of compress_bond.
+__host__ __device__ inline long compress_block(int Dmax) { return (2L * Dmax + 1) * Dmax; }
+// Largest bond whose two work matrices, singular values and their order fit the LDS (160 KB per CU).
+constexpr int COMPRESS_LDS_D = 64;
 
 // Walkers first .. first+gridDim-1 (population order) to bond targets[b];
 // afterwards sites 1..L-1 are right-orthonormal and site 0 is scaled to unit
 // norm (the LeftNormalize of Walker::setOverlap, Walker.cpp:54-66, up to gauge).
-template <typename T>
+// SM: the work matrices in LDS.
+template <typename T, bool SM>
 __global__ __launch_bounds__(MQE_NT) void compress_kernel(int L, Pool P, int first, const int *targets, char *scr,
                                                           long scr_bytes, int Dmax) {
     const int b = first + blockIdx.x;
@@ -173,13 +279,16 @@ __global__ __launch_bounds__(MQE_NT) void compress_kernel(int L, Pool P, int fir
     for (int k = threadIdx.x; k <= L; k += MQE_NT) wv[k] = P.wvd[(size_t)slot * (L + 1) + k];
     __syncthreads();
     T *phi = (T *)P.phi + (size_t)slot * P.wflat;
-    const long n2 = 4L * Dmax * Dmax;
-    double *X = (double *)(scr + (size_t)blockIdx.x * scr_bytes), *V = X + n2, *sig = V + n2;
+    extern __shared__ double compress_lds[];
+    double *X = SM ? compress_lds : (double *)(scr + (size_t)blockIdx.x * scr_bytes);
+    double *Y = X + compress_block(Dmax), *sig = Y + compress_block(Dmax);
     int *ord = (int *)(sig + 2 * Dmax);
     const int D = targets[b];
     if (D < 1) return;  // walker left as it is
-    for (int k = 0; k < L - 1; ++k) compress_bond(P, phi, wv, k, D, true, X, V, sig, ord, &flag);
-    for (int k = L - 2; k >= 0; --k) compress_bond(P, phi, wv, k, D, false, X, V, sig, ord, &flag);
+    for (int q = 0; q < 2 * (L - 1); ++q) {
+        const bool right = q < L - 1;
+        compress_bond<T, SM>(P, phi, wv, right ? q : 2 * (L - 1) - 1 - q, D, right, X, Y, sig, ord, &flag, red);
+    }
     const int w1 = wv[1];
     double s2 = 0.0;
     for (int e = threadIdx.x; e < 2 * w1; e += MQE_NT) {
@@ -1821,26 +1930,34 @@ int mqe_compress_walkers(mqe_engine *e, const int *targets) {
     ECHK(refresh_n(e));
     const int n = e->n_host, L = e->L;
     const int Dmax = e->Dw;
-    // per walker: X and V ((2 Dmax)^2 doubles each), Schmidt values and their order
-    const long scr_bytes = ((8L * (2 * 4L * Dmax * Dmax + 2 * Dmax) + 4L * 2 * Dmax) + 255) & ~255L;
-    const int chunk = std::max(1, std::min(n, (int)std::min(1024L, (1L << 30) / scr_bytes)));
+    // per walker: two work matrices, singular values and their order; in LDS up to
+    // Dmax = 64 (one launch, no scratch), beyond that in chunks of global scratch
+    const long work = ((8L * (2 * compress_block(Dmax) + 2 * Dmax) + 4L * 2 * Dmax) + 255) & ~255L;
+    const bool sm = Dmax <= COMPRESS_LDS_D;
+    const int chunk = sm ? n : std::max(1, std::min(n, (int)std::min(1024L, (1L << 30) / work)));
     char *scr = nullptr;
     int *dt = nullptr;
-    HIPCHK(hipMalloc((void **)&scr, (size_t)scr_bytes * chunk));
+    if (!sm) HIPCHK(hipMalloc((void **)&scr, (size_t)work * chunk));
     HIPCHK(hipMalloc((void **)&dt, sizeof(int) * n));
     HIPCHK(hipMemcpy(dt, targets, sizeof(int) * n, hipMemcpyHostToDevice));
     Pool P = make_pool(e, nullptr);
+    auto launch = [&](auto kernel, int f) -> hipError_t {
+        if (sm) {
+            const hipError_t r = hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                     (int)work);
+            if (r != hipSuccess) return r;
+        }
+        hipLaunchKernelGGL(kernel, dim3(chunk), dim3(MQE_NT), sm ? (size_t)work : 0, e->stream, L, P, f, dt, scr, work,
+                           Dmax);
+        return hipGetLastError();
+    };
     for (int f = 0; f < n; f += chunk) {
-        if (e->fp32)
-            hipLaunchKernelGGL(compress_kernel<float>, dim3(chunk), dim3(MQE_NT), 0, e->stream, L, P, f, dt, scr,
-                               scr_bytes, Dmax);
-        else
-            hipLaunchKernelGGL(compress_kernel<double>, dim3(chunk), dim3(MQE_NT), 0, e->stream, L, P, f, dt, scr,
-                               scr_bytes, Dmax);
-        HIPCHK(hipGetLastError());
+        if (e->fp32) HIPCHK(sm ? launch(compress_kernel<float, true>, f) : launch(compress_kernel<float, false>, f));
+        else HIPCHK(sm ? launch(compress_kernel<double, true>, f) : launch(compress_kernel<double, false>, f));
     }
     HIPCHK(hipStreamSynchronize(e->stream));
-    (void)hipFree(scr);
+    if (scr) (void)hipFree(scr);
+    scr = nullptr;
     // overlaps with the trial (transfer matrices), then the sign convention
     const int Do = std::max(e->Dw, e->Dt);
     const size_t tsz = e->fp32 ? sizeof(float) : sizeof(double);
