@@ -517,33 +517,46 @@ __device__ __forceinline__ void apply_op(const Ctx<T, CH> &C, int k, const doubl
 // LQ of site k (w_k x 2 w_{k+1}) in FP64: phi_k <- Q (right-orthonormal),
 // phi_{k-1} <- phi_{k-1} Lmat, then R_k = sum_t T_k[t] R_{k+1} Q[t]^T.
 // Leaves V (all four blocks) computed for bond k.
+// The factorisation is a serial chain of column steps; it runs with every
+// column in registers where the site fits (at most 128 x 64, reflectors in LDS)
+// and over columns in LDS and memory above.  One step of 200 walkers of a 15-site
+// ring in a field at D = 20 (two sweeps of LQ): 2121 us with the columns in LDS,
+// 1634 us in registers; 128 walkers of 16 sites at D = 16 in FP64, where one or
+// two walkers a step take this sweep and the others wait: 1230 and 1042 us.
 template <typename T, bool CH>
 __device__ __forceinline__ void lq_site(const Ctx<T, CH> &C, int k) {
     const int wk = C.wv[k], wn = C.wv[k + 1], wp = C.wv[k - 1];
     const int m = 2 * wn, n = wk;
-    // the FP64 factorisation's sequential column steps are latency-bound: the
-    // trailing columns (which receive most of the updates) live in LDS, as
-    // many as fit, the rest in the global scratch
-    double *R = C.ds + C.sl.RQ;
-    double *tau = C.qlds ? C.qlds : C.ds + C.sl.TAU;
-    int nl = 0;
-    if (C.qlds) nl = min(n, (int)((C.qlds_doubles - C.S->Dw) / m));
-    const QRCols col{C.ds + C.sl.AQ, C.qlds ? C.qlds + C.S->Dw : nullptr, m, n - nl};
     T *ph = C.site(k);
-    for (int e = threadIdx.x; e < m * n; e += MQE_NT) {
-        const int r = e % m, c = e / m;
-        col(c)[r] = (double)ph[c + (size_t)wk * r];
-    }
-    __syncthreads();
-    householder_qr(col, n, R, tau);
-    for (int e = threadIdx.x; e < m * n; e += MQE_NT) {
-        const int r = e % m, c = e / m;
-        ph[c + (size_t)wk * r] = (T)col(c)[r];
-    }
     T *LM = C.ts + C.sl.LM;
-    for (int e = threadIdx.x; e < n * n; e += MQE_NT) {
-        const int a = e % n, b = e / n;
-        LM[e] = (T)R[b + (size_t)n * a];
+    if (C.qlds && n <= m && m <= QR_REGS_M && n <= QR_REGS_N && (long)m * n + C.S->Dw <= C.qlds_doubles) {
+        qr_in_regs(
+            m, n, C.qlds + C.S->Dw, C.qlds, true, [&](int r, int c) { return (double)ph[c + (size_t)wk * r]; },
+            [&](int r, int c, double x) {
+                LM[c + (size_t)n * r] = (T)x;
+                if (r != c) LM[r + (size_t)n * c] = T(0);
+            },
+            [&](int r, int c, double x) { ph[c + (size_t)wk * r] = (T)x; });
+    } else {
+        double *R = C.ds + C.sl.RQ;
+        double *tau = C.qlds ? C.qlds : C.ds + C.sl.TAU;
+        int nl = 0;
+        if (C.qlds) nl = min(n, (int)((C.qlds_doubles - C.S->Dw) / m));
+        const QRCols col{C.ds + C.sl.AQ, C.qlds ? C.qlds + C.S->Dw : nullptr, m, n - nl};
+        for (int e = threadIdx.x; e < m * n; e += MQE_NT) {
+            const int r = e % m, c = e / m;
+            col(c)[r] = (double)ph[c + (size_t)wk * r];
+        }
+        __syncthreads();
+        householder_qr(col, n, R, tau);
+        for (int e = threadIdx.x; e < m * n; e += MQE_NT) {
+            const int r = e % m, c = e / m;
+            ph[c + (size_t)wk * r] = (T)col(c)[r];
+        }
+        for (int e = threadIdx.x; e < n * n; e += MQE_NT) {
+            const int a = e % n, b = e / n;
+            LM[e] = (T)R[b + (size_t)n * a];
+        }
     }
     __syncthreads();
     // push Lmat into the left neighbour
@@ -889,18 +902,9 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
 
     set_one(C.Lk(0));
 
-    if (flags & F_PREP) {
-        for (int k = 0; k < L - 1; ++k) advance_L(C, k);
-        double On, Ou;
-        const double e = energy_sweep(C, &On, &Ou, true);
-        if (threadIdx.x == 0) {
-            P.EL[slot] = e / O;  // stored overlap, MPSQMC2.cpp:447 / Walker.cpp:72-77
-            P.O[slot] = On;
-            P.since[slot] = 0;
-        }
-        return;
-    }
-
+    const bool prep = flags & F_PREP;
+    int p = 0;  // left environments L_k are valid for k <= p
+    if (!prep) {
     // ---------------- propagation (MPSQMC2.cpp:532-600) ----------------
     if (S.h != 0.0) {
         apply_field_everywhere(C);
@@ -908,9 +912,9 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
     }
     // The walker is not normalised between couplings: the sampled operator of
     // the right site is scaled so that the overlap stays O (see the file
-    // header), and the energy sweep takes the norm.  p: left environments L_k
-    // are valid for k <= p; rv: right environments R_k for k >= rv.
-    int p = 0, rv = 1;
+    // header), and the energy sweep takes the norm.  rv: right environments R_k are
+    // valid for k >= rv.
+    int rv = 1;
     for (int c = 0; c < S.nC; ++c) {
         const int i = S.first[c], j = S.second[c];
         // the left environments up to L_i and the right ones down to R_{j+1}: two
@@ -1026,20 +1030,27 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
         apply_field_everywhere(C);
         p = 0;
     }
+    }
     while (p < L - 1) {
         advance_L(C, p);
         ++p;
     }
     // ---------------- local energy (Walker.cpp:72-77) ----------------
+    // (one energy sweep for both kinds of call: a second inlined copy would only
+    // double the kernel's code)
     double On, Ou;
-    const bool canon = canon_walker(ctl, slot, P.since[slot]);
+    const bool canon = prep || canon_walker(ctl, slot, P.since[slot]);
     const double e = energy_sweep(C, &On, &Ou, canon);
     if (threadIdx.x == 0) {
         P.since[slot] = canon ? 0 : P.since[slot] + 1;
-        P.w[slot] = w;
         P.O[slot] = On;
-        P.EL[slot] = e / Ou;
-        if (!isfinite(w)) atomicOr(P.status, 2);
+        if (prep) {
+            P.EL[slot] = e / O;  // stored overlap, MPSQMC2.cpp:447 / Walker.cpp:72-77
+        } else {
+            P.w[slot] = w;
+            P.EL[slot] = e / Ou;
+            if (!isfinite(w)) atomicOr(P.status, 2);
+        }
     }
 }
 }  // namespace mqe
