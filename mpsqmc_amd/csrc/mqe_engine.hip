@@ -891,7 +891,12 @@ static int launch_walker_any(mqe_engine *e, const double *u, int flags) {
             if (r != MQE_OK) return r;
         }
         if (!collect) P.lab = nullptr;
-        t32::launch_walker32(wl, e->sys, P, e->d_t32N, e->d_t32T, flags, learn);
+        // bonds up to 16: one wave per walker in 16 x 16 tiles, at D = 8 twice the rate
+        // of the four-wave 32 x 32 kernel; the learned proposal is only in the latter
+        if (!learn && e->Dt <= t16::MAXD && e->Dw <= t16::MAXD)
+            t16::launch_walker16(wl, e->sys, P, e->d_t32N, e->d_t32T, flags);
+        else
+            t32::launch_walker32(wl, e->sys, P, e->d_t32N, e->d_t32T, flags, learn);
         HIPCHK(hipGetLastError());
         if (collect) {
             hipLaunchKernelGGL(advance_samples_kernel, dim3(1), dim3(64), 0, e->stream, e->d_n, e->nC, e->d_nsamp,

@@ -152,6 +152,12 @@ void launch_walker32(const WalkerLaunch &l, const Sys &S, const Pool &P, const f
 hipError_t lds_attr32();
 }  // namespace t32
 
+namespace t16 {
+// the same storage and trial blocks; bonds up to MAXD, no learned proposal
+constexpr int MAXD = 16;
+void launch_walker16(const WalkerLaunch &l, const Sys &S, const Pool &P, const float *TN, const float *TT, int flags);
+}  // namespace t16
+
 }  // namespace mqe
 
 #endif
