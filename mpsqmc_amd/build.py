@@ -12,7 +12,7 @@ ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libmqe.so")
 
-SOURCES = ["mqe_walker_f32c.hip", "mqe_walker_f32.hip", "mqe_walker_f64.hip",
+SOURCES = ["mqe_walker_f32c.hip", "mqe_walker_f64c.hip", "mqe_walker_f32.hip", "mqe_walker_f64.hip",
            "mqe_walker_tile.hip", "mqe_walker_small.hip", "mqe_engine.hip", "mqe_mlp.hip",
            "mqe_noalloc.hip", "mqe_host.cpp", "mqe_dmrg.cpp", "mpsqmc.cpp"]
 WALK = os.path.join(HERE, "mpsqmc_walk")

@@ -497,11 +497,12 @@ __device__ __forceinline__ void gemm(int m, int n, int k, const T *A, int lda, c
 // TB: B_f stored n1 x k1 (op(B) = B^T).  TC: C stored m1 x mD (op(C) = C^T,
 // contiguous along the inner index), else mD x m1.  All matrices column-major.
 // ---------------------------------------------------------------------------
+template <typename T>
 struct ChainOps {
-    const float *A;      // m1 x k1, leading dimension lda
-    const float *B[2];   // B_f
-    const float *C[2];   // C_f (ND = 1) or C_d (ND = 2)
-    float *D[2];         // D_d, mD x n1, leading dimension ldd
+    const T *A;      // m1 x k1, leading dimension lda
+    const T *B[2];   // B_f
+    const T *C[2];   // C_f (ND = 1) or C_d (ND = 2)
+    T *D[2];         // D_d, mD x n1, leading dimension ldd
 };
 
 typedef float v16f_c __attribute__((ext_vector_type(16)));
@@ -519,11 +520,17 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, BUF_RANGE, 0x00020000);
 }
 // (the b32 / b128 builtins move raw 32-bit words: bit casts, not conversions)
-__device__ __forceinline__ float buf_ld(__amdgpu_buffer_rsrc_t r, int voff) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
+template <typename T = float>
+__device__ __forceinline__ T buf_ld(__amdgpu_buffer_rsrc_t r, int voff) {
+    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
+    else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
 }
 __device__ __forceinline__ void buf_st(float v, __amdgpu_buffer_rsrc_t r, int voff, int imm) {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, voff, imm, 0);
+}
+__device__ __forceinline__ void buf_st(double v, __amdgpu_buffer_rsrc_t r, int voff, int imm) {
+    typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, voff, imm, 0);
 }
 __device__ __forceinline__ void buf_ld4(__amdgpu_buffer_rsrc_t r, int voff, float *v) {
     const float4 x = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
@@ -551,7 +558,7 @@ __device__ __forceinline__ int chain2(int wave0, int nu, int m1, int n1, int k1,
         const int qi = it % nq, rest = it / nq;
         const int u = rest / nstrip, c0 = (rest - u * nstrip) * 32;
         const bool do0 = nq == 1 || qi == 0, do1 = twoD && (nq == 1 || qi == 1);  // D row tiles of this item
-        const ChainOps op = get(u);
+        const ChainOps<float> op = get(u);
         // the lane coordinates as opaque values inside the loops: the per-element
         // offsets below are then formed next to their loads instead of being
         // hoisted out of the loops and held in registers throughout
@@ -675,56 +682,84 @@ __device__ __forceinline__ int chain2(int wave0, int nu, int m1, int n1, int k1,
 // (a bond of 48 in three 16-column strips re-reads A and C three times and
 // measured 20 % slower than two 32-column strips).
 // qsplit: the D row tiles 0-1 and 2-3 are separate items.
-typedef float v4f_c __attribute__((ext_vector_type(4)));
+// FP64 (v_mfma_f64_16x16x4f64) takes all bonds up to 64 this way.  Its
+// accumulator slot e of lane (c, g) holds row g + 4e, so MFMA e of F tile t in
+// the second chain takes rows 16t + g + 4e.  The general products' vector-unit
+// loops read both operands of every multiplication from memory and pass the
+// intermediate through it; 48 walkers of the 4x4 torus at D = 20 took 18.4 ms a
+// step with them and take 7.6 ms with the chains; 128 walkers of a 16-site chain at
+// D = 16: 1042 and 739 us.
+template <typename T>
+struct Chain16;
+template <>
+struct Chain16<float> {
+    typedef float V4 __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ V4 mfma(float a, float b, V4 c) {
+        return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int g, int e) { return 4 * g + e; }
+    static constexpr int ROW_G = 4, ROW_E = 1;  // row = ROW_G g + ROW_E e
+};
+template <>
+struct Chain16<double> {
+    typedef double V4 __attribute__((ext_vector_type(4)));
+    static __device__ __forceinline__ V4 mfma(double a, double b, V4 c) {
+        return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+    }
+    static __device__ __forceinline__ int row(int g, int e) { return g + 4 * e; }
+    static constexpr int ROW_G = 1, ROW_E = 4;
+};
 
-__device__ __forceinline__ v4f_c mfma16(float a, float b, v4f_c c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-
-template <bool TB, bool TC, int NF, int ND, class Get>
+template <bool TB, bool TC, int NF, int ND, typename T, class Get>
 __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int k1, int mD, int lda, int ldb, int ldc,
                                          int ldd, bool qsplit, Get get) {
+    typedef Chain16<T> CT;
+    typedef typename CT::V4 V4;
+    constexpr int SZ = sizeof(T);
     static_assert(ND == 1 || NF == 1, "two outputs take one intermediate");
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int MT = (m1 + 15) >> 4, QT = (mD + 15) >> 4;  // F and D row tiles (<= 4)
     const int nq = qsplit && QT > 2 ? 2 : 1;
     const int nstrip = (n1 + 15) >> 4, nitems = nu * nstrip * nq;
-    const int sa = 4 * lda, sb = TB ? 4 * ldb : 4;  // bytes per k step of A and op(B)
+    const int sa = SZ * lda, sb = TB ? SZ * ldb : SZ;  // bytes per k step of A and op(B)
     const int kf = k1 & ~15;
 #pragma nounroll
     for (int it = (w - wave0 + 2 * MQE_WAVES) % MQE_WAVES; it < nitems; it += MQE_WAVES) {
         const int qi = it % nq, rest = it / nq;
         const int u = rest / nstrip, c0 = (rest - u * nstrip) * 16;
         const int q0 = nq == 1 ? 0 : 2 * qi, q1 = nq == 1 ? QT : min(QT, 2 * qi + 2);  // D row tiles of this item
-        const ChainOps op = get(u);
+        const ChainOps<T> op = get(u);
         int c = lane & 15, g = lane >> 4;
-        v4f_c D[4];
+        V4 D[4];
 #pragma nounroll
         for (int f = 0; f < NF; ++f) {
             asm volatile("" : "+v"(c), "+v"(g));
             const int col = min(c0 + c, n1 - 1);
-            const int vB = TB ? 4 * col : 4 * ldb * col;
+            const int vB = TB ? SZ * col : SZ * ldb * col;
             // ---- first chain: the F_f strip (16 columns), up to four 16-row tiles ----
-            v4f_c F[4];
+            V4 F[4];
 #pragma unroll
-            for (int t = 0; t < 4; ++t) F[t] = v4f_c{0.f, 0.f, 0.f, 0.f};
+            for (int t = 0; t < 4; ++t) F[t] = V4{0, 0, 0, 0};
             const auto rA = buf_rsrc(op.A), rB = buf_rsrc(op.B[f]);
+            // the last, partial slice takes k = kf + 4q + g, so that a step wholly past k1 is left out
             auto slice = [&](int k0, bool tail) {
-                const int kl = k0 + 4 * g;
-                float a[4][4], bv[4];
+                T a[4][4], bv[4];
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    const bool ok = !tail || kl + q < k1;
-                    bv[q] = buf_ld(rB, ok ? vB + sb * (kl + q) : BUF_OOB);
+                    const int k = tail ? k0 + 4 * q + g : k0 + 4 * g + q;
+                    const bool ok = !tail || k < k1;
+                    bv[q] = buf_ld<T>(rB, ok ? vB + sb * k : BUF_OOB);
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
-                        a[t][q] = t < MT ? buf_ld(rA, ok ? 4 * min(16 * t + c, m1 - 1) + sa * (kl + q) : BUF_OOB) : 0.f;
+                        a[t][q] = t < MT ? buf_ld<T>(rA, ok ? SZ * min(16 * t + c, m1 - 1) + sa * k : BUF_OOB) : T(0);
                 }
 #pragma unroll
-                for (int q = 0; q < 4; ++q)
+                for (int q = 0; q < 4; ++q) {
+                    if (tail && k0 + 4 * q >= k1) break;
 #pragma unroll
                     for (int t = 0; t < 4; ++t)
-                        if (t < MT) F[t] = mfma16(a[t][q], bv[q], F[t]);
+                        if (t < MT) F[t] = CT::mfma(a[t][q], bv[q], F[t]);
+                }
             };
 #pragma nounroll
             for (int k0 = 0; k0 < kf; k0 += 16) slice(k0, false);
@@ -734,35 +769,35 @@ __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int 
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
                     for (int e = 0; e < 4; ++e)
-                        if (16 * t + 4 * g + e >= m1) F[t][e] = 0.f;
+                        if (16 * t + CT::row(g, e) >= m1) F[t][e] = T(0);
             }
             // ---- second chain: D_d (+)= op(C) F_f, 16-row tile by tile ----
 #pragma nounroll
             for (int d = 0; d < ND; ++d) {
                 asm volatile("" : "+v"(c), "+v"(g));
-                const float *Cp = op.C[ND == 1 ? f : d];
+                const T *Cp = op.C[ND == 1 ? f : d];
                 const auto rC = buf_rsrc(Cp);
-                const bool vecC = TC && (m1 & 3) == 0 && (ldc & 3) == 0 && aligned16(Cp, Cp, 0, 0);
+                const bool vecC = TC && SZ == 4 && (m1 & 3) == 0 && (ldc & 3) == 0 && (((uintptr_t)Cp) & 15u) == 0;
                 if (ND == 2 || f == 0) {
 #pragma unroll
-                    for (int qd = 0; qd < 4; ++qd) D[qd] = v4f_c{0.f, 0.f, 0.f, 0.f};
+                    for (int qd = 0; qd < 4; ++qd) D[qd] = V4{0, 0, 0, 0};
                 }
 #pragma unroll
                 for (int qd = 0; qd < 4; ++qd) {
                     if (qd < q0 || qd >= q1) continue;
                     const int row = min(16 * qd + c, mD - 1);
-                    float cv[4][4];
+                    T cv[4][4];
 #pragma unroll
                     for (int t = 0; t < 4; ++t) {
                         if (t >= MT) continue;
-                        if (TC && vecC) {
+                        if (TC && SZ == 4 && vecC) {
                             // a run at or beyond m1 meets zero rows of F: any values of C do
-                            buf_ld4(rC, 4 * (ldc * row + min(16 * t + 4 * g, m1 - 4)), cv[t]);
+                            buf_ld4(rC, 4 * (ldc * row + min(16 * t + 4 * g, m1 - 4)), (float *)cv[t]);
                         } else {
 #pragma unroll
                             for (int e = 0; e < 4; ++e) {
-                                const int k = min(16 * t + 4 * g + e, m1 - 1);
-                                cv[t][e] = buf_ld(rC, TC ? 4 * (ldc * row + k) : 4 * (row + ldc * k));
+                                const int k = min(16 * t + CT::row(g, e), m1 - 1);
+                                cv[t][e] = buf_ld<T>(rC, TC ? SZ * (ldc * row + k) : SZ * (row + ldc * k));
                             }
                         }
                     }
@@ -770,19 +805,22 @@ __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int 
                     for (int t = 0; t < 4; ++t) {
                         if (t >= MT) continue;
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) D[qd] = mfma16(cv[t][e], F[t][e], D[qd]);
+                        for (int e = 0; e < 4; ++e) {
+                            if (CT::ROW_G == 1 && 16 * t + 4 * e >= m1) break;  // rows 4e .. 4e + 3 of F are zero
+                            D[qd] = CT::mfma(cv[t][e], F[t][e], D[qd]);
+                        }
                     }
                 }
                 if (f == NF - 1) {
-                    // row 16 qd + 4g + e of column c0 + c; outside D the store is dropped
-                    const int vd = c0 + c < n1 ? 4 * (ldd * (c0 + c) + 4 * g) : BUF_OOB;
+                    // row 16 qd + row(g, e) of column c0 + c; outside D the store is dropped
+                    const int vd = c0 + c < n1 ? SZ * (ldd * (c0 + c) + CT::ROW_G * g) : BUF_OOB;
                     const auto rD = buf_rsrc(op.D[d]);
 #pragma unroll
                     for (int qd = 0; qd < 4; ++qd) {
                         if (qd < q0 || qd >= q1) continue;
 #pragma unroll
                         for (int e = 0; e < 4; ++e)
-                            buf_st(D[qd][e], rD, 16 * qd + 4 * g + e < mD ? vd : BUF_OOB, 4 * (16 * qd + e));
+                            buf_st(D[qd][e], rD, 16 * qd + CT::row(g, e) < mD ? vd : BUF_OOB, SZ * (16 * qd + CT::ROW_E * e));
                     }
                 }
             }

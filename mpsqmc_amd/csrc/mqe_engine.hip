@@ -729,7 +729,7 @@ struct mqe_engine {
     bool tile32 = false;   // FP32 MFMA path for NN chains with bonds <= 32, h = 0
     float *d_t32N = nullptr, *d_t32T = nullptr;
     float *d_trialT = nullptr;  // chained general kernel: every T_k[s] transposed
-    bool chained = false;       // the general kernel with chained FP32 products (bonds <= 64)
+    bool chained = false;       // the general kernel with chained products (bonds <= 64)
     hipStream_t stream = nullptr;
     std::vector<int> tvd, wmax;
     std::vector<long> toff, woff, eoff, moff;
@@ -902,8 +902,9 @@ static int launch_walker_any(mqe_engine *e, const double *u, int flags) {
             hipLaunchKernelGGL(advance_samples_kernel, dim3(1), dim3(64), 0, e->stream, e->d_n, e->nC, e->d_nsamp,
                                e->max_samples);
         }
-    } else if (e->chained) launch_walker_f32_chained(wl, e->sys, P, (const float *)e->d_trial, flags);
+    } else if (e->chained && e->fp32) launch_walker_f32_chained(wl, e->sys, P, (const float *)e->d_trial, flags);
     else if (e->fp32) launch_walker_f32(wl, e->sys, P, (const float *)e->d_trial, flags);
+    else if (e->chained) launch_walker_f64_chained(wl, e->sys, P, (const double *)e->d_trial, flags);
     else launch_walker_f64(wl, e->sys, P, (const double *)e->d_trial, flags);
     HIPCHK(hipGetLastError());
     return MQE_OK;
@@ -1163,9 +1164,9 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
     }
     {
         const char *noch = getenv("MQE_NO_CHAIN");
-        e->chained = e->fp32 && !e->tile32 && e->Dt <= 64 && e->Dw <= 64 && !(noch && noch[0] == '1');
+        e->chained = !e->tile32 && e->Dt <= 64 && e->Dw <= 64 && !(noch && noch[0] == '1');
     }
-    if (e->chained) {
+    if (e->chained && e->fp32) {
         // the trial with every T_k[s] transposed (t_{k+1} x t_k), same offsets:
         // the chained products read trial operands along the inner index
         std::vector<float> tt((size_t)tsize);
@@ -1215,6 +1216,7 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
             CK(lds_attr_f32_chained(need));
             CK(lds_attr_f32(need));
             CK(lds_attr_f64(need));
+            CK(lds_attr_f64_chained(need));
         }
     }
     const int nC = n_couplings;

@@ -11,7 +11,7 @@ namespace mqe {
 // ---------------------------------------------------------------------------
 // per-walker context
 // ---------------------------------------------------------------------------
-// CH: the FP32 products are chained in registers (chain2); the host selects
+// CH: the products are chained in registers (chain2, chain2_16); the host selects
 // this instance only when every trial and walker bond is at most 64.
 template <typename T, bool CH>
 struct Ctx {
@@ -32,7 +32,14 @@ struct Ctx {
 
     __device__ T *site(int k) const { return phi + woff[k]; }
     __device__ const T *tsite(int k) const { return trial + S->toff[k]; }
-    __device__ const float *tsiteT(int k) const { return trialT + S->toff[k]; }
+    // site k of the trial as the second operand of a product T_k[s] F: FP32 takes
+    // the transposed copy (four values along the inner index per load), FP64 the
+    // plain one (its inner index is strided over the lanes)
+    static constexpr bool TRT = sizeof(T) == sizeof(float);
+    __device__ const T *tsiteR(int k) const {
+        if constexpr (TRT) return trialT + S->toff[k];
+        else return tsite(k);
+    }
 
     __device__ T *Lk(int k) const { return Lenv + eoff[k]; }
     __device__ T *Rk(int k) const { return Renv + eoff[k]; }
@@ -51,29 +58,33 @@ __device__ __forceinline__ int issue_G(const Ctx<T, CH> &C, int i, const T *Lenv
                                        int wave0) {
     if constexpr (CH) {
         const int ti = C.tv[i], tn = C.tv[i + 1], wi = C.wv[i], wn = C.wv[i + 1];
-        const float *Ti = (const float *)C.tsite(i), *ph = (const float *)C.site(i);
+        const T *Ti = C.tsite(i), *ph = C.site(i);
         auto unit = [&](int u) {
             const int sp = u >> 1, s = u & 1;
-            ChainOps o;
-            o.A = (const float *)Lenv_i;
+            ChainOps<T> o;
+            o.A = Lenv_i;
             o.B[0] = o.B[1] = ph + (size_t)s * wi * wn;
             o.C[0] = o.C[1] = Ti + (size_t)sp * ti * tn;
-            o.D[0] = o.D[1] = (float *)out + (size_t)sp * ssp + (size_t)s * ss;
+            o.D[0] = o.D[1] = out + (size_t)sp * ssp + (size_t)s * ss;
             return o;
         };
-        if (wn < 32) return chain2_16<false, true, 1, 1>(wave0, 4, ti, wn, wi, tn, ti, wi, ti, ldo, false, unit);
-        if (wn > 32)
-            return chain2<false, true, 1, 2>(wave0, 2, ti, wn, wi, tn, ti, wi, ti, ldo, false, [&](int s) {
-                ChainOps o;
-                o.A = (const float *)Lenv_i;
-                o.B[0] = o.B[1] = ph + (size_t)s * wi * wn;
-                o.C[0] = Ti;
-                o.C[1] = Ti + (size_t)ti * tn;
-                o.D[0] = (float *)out + (size_t)s * ss;
-                o.D[1] = (float *)out + (size_t)ssp + (size_t)s * ss;
-                return o;
-            });
-        return chain2<false, true, 1, 1>(wave0, 4, ti, wn, wi, tn, ti, wi, ti, ldo, false, unit);
+        auto both = [&](int s) {
+            ChainOps<T> o;
+            o.A = Lenv_i;
+            o.B[0] = o.B[1] = ph + (size_t)s * wi * wn;
+            o.C[0] = Ti;
+            o.C[1] = Ti + (size_t)ti * tn;
+            o.D[0] = out + (size_t)s * ss;
+            o.D[1] = out + (size_t)ssp + (size_t)s * ss;
+            return o;
+        };
+        if constexpr (sizeof(T) == sizeof(float)) {
+            if (wn > 32) return chain2<false, true, 1, 2>(wave0, 2, ti, wn, wi, tn, ti, wi, ti, ldo, false, both);
+            if (wn == 32) return chain2<false, true, 1, 1>(wave0, 4, ti, wn, wi, tn, ti, wi, ti, ldo, false, unit);
+        } else {
+            if (wn > 16) return chain2_16<false, true, 1, 2, T>(wave0, 2, ti, wn, wi, tn, ti, wi, ti, ldo, false, both);
+        }
+        return chain2_16<false, true, 1, 1, T>(wave0, 4, ti, wn, wi, tn, ti, wi, ti, ldo, false, unit);
     }
     return wave0;
 }
@@ -82,31 +93,36 @@ __device__ __forceinline__ int issue_G(const Ctx<T, CH> &C, int i, const T *Lenv
 template <typename T, bool CH>
 __device__ __forceinline__ int issue_V(const Ctx<T, CH> &C, int j, int wave0) {
     if constexpr (CH) {
-        const int tj = C.tv[j], tn = C.tv[j + 1], wj = C.wv[j], wn = C.wv[j + 1];
-        const float *R = (const float *)C.Rk(j + 1), *ph = (const float *)C.site(j), *TTj = C.tsiteT(j);
-        float *V = (float *)(C.ts + C.sl.V);
+        constexpr bool TRT = Ctx<T, CH>::TRT;
+        const int tj = C.tv[j], tn = C.tv[j + 1], wj = C.wv[j], wn = C.wv[j + 1], ldc = TRT ? tn : tj;
+        const T *R = C.Rk(j + 1), *ph = C.site(j), *TTj = C.tsiteR(j);
+        T *V = C.ts + C.sl.V;
         auto unit = [&](int u) {
             const int tp = u >> 1, t = u & 1;
-            ChainOps o;
+            ChainOps<T> o;
             o.A = R;
             o.B[0] = o.B[1] = ph + (size_t)t * wj * wn;
             o.C[0] = o.C[1] = TTj + (size_t)tp * tj * tn;
             o.D[0] = o.D[1] = V + (size_t)tp * tj * 2 * wj + (size_t)t * tj * wj;
             return o;
         };
-        if (wj < 32) return chain2_16<true, true, 1, 1>(wave0, 4, tn, wj, wn, tj, tn, wj, tn, tj, false, unit);
-        if (wj > 32)
-            return chain2<true, true, 1, 2>(wave0, 2, tn, wj, wn, tj, tn, wj, tn, tj, false, [&](int t) {
-                ChainOps o;
-                o.A = R;
-                o.B[0] = o.B[1] = ph + (size_t)t * wj * wn;
-                o.C[0] = TTj;
-                o.C[1] = TTj + (size_t)tj * tn;
-                o.D[0] = V + (size_t)t * tj * wj;
-                o.D[1] = V + (size_t)tj * 2 * wj + (size_t)t * tj * wj;
-                return o;
-            });
-        return chain2<true, true, 1, 1>(wave0, 4, tn, wj, wn, tj, tn, wj, tn, tj, false, unit);
+        auto both = [&](int t) {
+            ChainOps<T> o;
+            o.A = R;
+            o.B[0] = o.B[1] = ph + (size_t)t * wj * wn;
+            o.C[0] = TTj;
+            o.C[1] = TTj + (size_t)tj * tn;
+            o.D[0] = V + (size_t)t * tj * wj;
+            o.D[1] = V + (size_t)tj * 2 * wj + (size_t)t * tj * wj;
+            return o;
+        };
+        if constexpr (sizeof(T) == sizeof(float)) {
+            if (wj > 32) return chain2<true, TRT, 1, 2>(wave0, 2, tn, wj, wn, tj, tn, wj, ldc, tj, false, both);
+            if (wj == 32) return chain2<true, TRT, 1, 1>(wave0, 4, tn, wj, wn, tj, tn, wj, ldc, tj, false, unit);
+        } else {
+            if (wj > 16) return chain2_16<true, TRT, 1, 2, T>(wave0, 2, tn, wj, wn, tj, tn, wj, ldc, tj, false, both);
+        }
+        return chain2_16<true, TRT, 1, 1, T>(wave0, 4, tn, wj, wn, tj, tn, wj, ldc, tj, false, unit);
     }
     return wave0;
 }
@@ -173,26 +189,28 @@ template <typename T, bool CH>
 __device__ __forceinline__ void carry_channels(const Ctx<T, CH> &C, int k, const T *src, T *dst, int nch = 4) {
     const int tk = C.tv[k], tn = C.tv[k + 1], wk = C.wv[k], wn = C.wv[k + 1];
     const T *Tk = C.tsite(k);
-    if constexpr (sizeof(T) == sizeof(float)) {
-        if constexpr (CH) {
-            const float *ph = (const float *)C.site(k);
-            auto unit = [&](int ch) {
-                ChainOps o;
-                o.A = (const float *)src + (size_t)ch * tk * wk;
-                o.B[0] = ph;
-                o.B[1] = ph + (size_t)wk * wn;
-                o.C[0] = (const float *)Tk;
-                o.C[1] = (const float *)Tk + (size_t)tk * tn;
-                o.D[0] = o.D[1] = (float *)dst + (size_t)ch * tn * wn;
-                return o;
-            };
-            if (wn < 32)
-                chain2_16<false, true, 2, 1>(0, nch, tk, wn, wk, tn, tk, wk, tk, tn, false, unit);
-            else
+    if constexpr (CH) {
+        const T *ph = C.site(k);
+        auto unit = [&](int ch) {
+            ChainOps<T> o;
+            o.A = src + (size_t)ch * tk * wk;
+            o.B[0] = ph;
+            o.B[1] = ph + (size_t)wk * wn;
+            o.C[0] = Tk;
+            o.C[1] = Tk + (size_t)tk * tn;
+            o.D[0] = o.D[1] = dst + (size_t)ch * tn * wn;
+            return o;
+        };
+        if constexpr (sizeof(T) == sizeof(float)) {
+            if (wn >= 32) {
                 chain2<false, true, 2, 1>(0, nch, tk, wn, wk, tn, tk, wk, tk, tn, false, unit);
-            __syncthreads();
-            return;
+                __syncthreads();
+                return;
+            }
         }
+        chain2_16<false, true, 2, 1, T>(0, nch, tk, wn, wk, tn, tk, wk, tk, tn, false, unit);
+        __syncthreads();
+        return;
     }
     T *Y = C.ts + C.sl.Y4;  // Y_ch = src_ch phi_k (tk x 2 wn), the four channels one after the other
     const long sy = (long)tk * 2 * wn;
@@ -345,19 +363,21 @@ template <typename T, bool CH>
 __device__ __forceinline__ int issue_L(const Ctx<T, CH> &C, int k, int wave0) {
     if constexpr (CH) {
         const int tk = C.tv[k], tn = C.tv[k + 1], wk = C.wv[k], wn = C.wv[k + 1];
-        const float *ph = (const float *)C.site(k), *Tk = (const float *)C.tsite(k);
+        const T *ph = C.site(k), *Tk = C.tsite(k);
         auto unit = [&](int) {
-            ChainOps o;
-            o.A = (const float *)C.Lk(k);
+            ChainOps<T> o;
+            o.A = C.Lk(k);
             o.B[0] = ph;
             o.B[1] = ph + (size_t)wk * wn;
             o.C[0] = Tk;
             o.C[1] = Tk + (size_t)tk * tn;
-            o.D[0] = o.D[1] = (float *)C.Lk(k + 1);
+            o.D[0] = o.D[1] = C.Lk(k + 1);
             return o;
         };
-        if (wn < 32) return chain2_16<false, true, 2, 1>(wave0, 1, tk, wn, wk, tn, tk, wk, tk, tn, true, unit);
-        return chain2<false, true, 2, 1>(wave0, 1, tk, wn, wk, tn, tk, wk, tk, tn, true, unit);
+        if constexpr (sizeof(T) == sizeof(float)) {
+            if (wn >= 32) return chain2<false, true, 2, 1>(wave0, 1, tk, wn, wk, tn, tk, wk, tk, tn, true, unit);
+        }
+        return chain2_16<false, true, 2, 1, T>(wave0, 1, tk, wn, wk, tn, tk, wk, tk, tn, true, unit);
     }
     return wave0;
 }
@@ -384,19 +404,23 @@ template <typename T, bool CH>
 __device__ __forceinline__ int issue_R(const Ctx<T, CH> &C, int k, int wave0) {
     if constexpr (CH) {
         const int tk = C.tv[k], tn = C.tv[k + 1], wk = C.wv[k], wn = C.wv[k + 1];
-        const float *ph = (const float *)C.site(k), *TTk = C.tsiteT(k);
+        constexpr bool TRT = Ctx<T, CH>::TRT;
+        const int ldc = TRT ? tn : tk;
+        const T *ph = C.site(k), *TTk = C.tsiteR(k);
         auto unit = [&](int) {
-            ChainOps o;
-            o.A = (const float *)C.Rk(k + 1);
+            ChainOps<T> o;
+            o.A = C.Rk(k + 1);
             o.B[0] = ph;
             o.B[1] = ph + (size_t)wk * wn;
             o.C[0] = TTk;
             o.C[1] = TTk + (size_t)tk * tn;
-            o.D[0] = o.D[1] = (float *)C.Rk(k);
+            o.D[0] = o.D[1] = C.Rk(k);
             return o;
         };
-        if (wk < 32) return chain2_16<true, true, 2, 1>(wave0, 1, tn, wk, wn, tk, tn, wk, tn, tk, true, unit);
-        return chain2<true, true, 2, 1>(wave0, 1, tn, wk, wn, tk, tn, wk, tn, tk, true, unit);
+        if constexpr (sizeof(T) == sizeof(float)) {
+            if (wk >= 32) return chain2<true, TRT, 2, 1>(wave0, 1, tn, wk, wn, tk, tn, wk, ldc, tk, true, unit);
+        }
+        return chain2_16<true, TRT, 2, 1, T>(wave0, 1, tn, wk, wn, tk, tn, wk, ldc, tk, true, unit);
     }
     return wave0;
 }
@@ -423,18 +447,20 @@ template <typename T, bool CH>
 __device__ __forceinline__ int issue_M(const Ctx<T, CH> &C, int k, int wave0) {
     if constexpr (CH) {
         const int wk = C.wv[k], wn = C.wv[k + 1];
-        const float *ph = (const float *)C.site(k), *Mn = (const float *)C.Mk(k + 1);
-        float *Mk = (float *)C.Mk(k);
+        const T *ph = C.site(k), *Mn = C.Mk(k + 1);
+        T *Mk = C.Mk(k);
         auto unit = [&](int) {
-            ChainOps o;
+            ChainOps<T> o;
             o.A = Mn;
             o.B[0] = o.C[0] = ph;
             o.B[1] = o.C[1] = ph + (size_t)wk * wn;
             o.D[0] = o.D[1] = Mk;
             return o;
         };
-        if (wk < 32) return chain2_16<true, false, 2, 1>(wave0, 1, wn, wk, wn, wk, wn, wk, wk, wk, false, unit);
-        return chain2<true, false, 2, 1>(wave0, 1, wn, wk, wn, wk, wn, wk, wk, wk, false, unit);
+        if constexpr (sizeof(T) == sizeof(float)) {
+            if (wk >= 32) return chain2<true, false, 2, 1>(wave0, 1, wn, wk, wn, wk, wn, wk, wk, wk, false, unit);
+        }
+        return chain2_16<true, false, 2, 1, T>(wave0, 1, wn, wk, wn, wk, wn, wk, wk, wk, false, unit);
     }
     return wave0;
 }

@@ -140,9 +140,11 @@ struct WalkerLaunch {
 void launch_walker_f32(const WalkerLaunch &l, const Sys &S, const Pool &P, const float *trial, int flags);
 void launch_walker_f32_chained(const WalkerLaunch &l, const Sys &S, const Pool &P, const float *trial, int flags);
 void launch_walker_f64(const WalkerLaunch &l, const Sys &S, const Pool &P, const double *trial, int flags);
+void launch_walker_f64_chained(const WalkerLaunch &l, const Sys &S, const Pool &P, const double *trial, int flags);
 hipError_t lds_attr_f32(size_t lds);
 hipError_t lds_attr_f32_chained(size_t lds);
 hipError_t lds_attr_f64(size_t lds);
+hipError_t lds_attr_f64_chained(size_t lds);
 
 namespace t32 {
 constexpr int MAXG_T32 = 256;  // grid points: four per lane of one wave

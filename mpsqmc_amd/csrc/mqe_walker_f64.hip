@@ -1,4 +1,4 @@
-// mqe_walker_f64.hip -- the general walker kernel, FP64.
+// mqe_walker_f64.hip -- the general walker kernel, FP64, bonds above 64.
 #include <hip/hip_runtime.h>
 
 #include "mqe_general.h"

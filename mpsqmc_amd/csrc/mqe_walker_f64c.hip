@@ -1,0 +1,17 @@
+// mqe_walker_f64c.hip -- the general walker kernel, FP64 with chained products, bonds up to 64.
+#include <hip/hip_runtime.h>
+
+#include "mqe_general.h"
+
+namespace mqe {
+
+void launch_walker_f64_chained(const WalkerLaunch &l, const Sys &S, const Pool &P, const double *trial, int flags) {
+    hipLaunchKernelGGL((walker_kernel<double, true>), dim3(l.grid), dim3(MQE_NT), l.lds, l.stream, S, P, trial, flags);
+}
+
+hipError_t lds_attr_f64_chained(size_t lds) {
+    return hipFuncSetAttribute((const void *)walker_kernel<double, true>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                               (int)lds);
+}
+
+}  // namespace mqe
