@@ -12,7 +12,7 @@
 // MFMA GEMM (v_mfma_f32_32x32x2f32) with the weights read from global memory
 // (80 KB at H = 128, L2-resident).  Training computes forward and backward of a
 // tile and writes the tile's gradient to its own slot; the Adam kernel sums the
-// slots in tile order (deterministic) and updates the parameters.
+// slots in a fixed order (deterministic) and updates the parameters.
 //
 // Parameter layout (column-major): W1 [H x n_in], b1 [H], W2 [H x H], b2 [H],
 // W3 [n_out x H], b3 [n_out].  Inputs are standardised with (x - x_mean) /
@@ -162,21 +162,46 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
     }
 }
 
-// Sum of the tile gradients (in tile order) and one Adam step.
-__global__ void adam_kernel(float *par, float *m, float *v, const float *gpart, int ntiles, long np, float lr,
-                            float b1, float b2, float eps, float c1, float c2, float *grad_out) {
-    for (long p = (long)blockIdx.x * blockDim.x + threadIdx.x; p < np; p += (long)gridDim.x * blockDim.x) {
-        float g = 0.f;
-        for (int t = 0; t < ntiles; ++t) g += gpart[(size_t)t * np + p];
-        if (grad_out) {
-            grad_out[p] = g;
-            continue;
+// Sum of the tile gradients (in a fixed order: wave w of a workgroup takes the
+// tiles congruent to w, the waves' sums are added in their order) and one Adam step.
+// What bounds it: memory, one pass over the tile gradients (22 MB for 16,384 rows
+// at H = 128).  A thread takes one parameter and keeps 16 tiles' loads in flight;
+// one thread per parameter over all tiles in turn, with 85 workgroups, waited for
+// 256 loads one after the other for 60 us: a loss_grad call from 287 to 230 us.
+constexpr int SUM_P = 64;  // parameters of a workgroup, one per lane
+__global__ __launch_bounds__(MQE_NT) void adam_kernel(float *par, float *m, float *v, const float *gpart, int ntiles,
+                                                      long np, float lr, float b1, float b2, float eps, float c1,
+                                                      float c2, float *grad_out) {
+    __shared__ float part[MQE_WAVES][SUM_P];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const long p = (long)blockIdx.x * SUM_P + lane;
+    float g = 0.f;
+    if (p < np) {
+        const float *src = gpart + p;
+        int t = w;
+        for (; t + 15 * MQE_WAVES < ntiles; t += 16 * MQE_WAVES) {
+            float x[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) x[q] = src[(size_t)(t + MQE_WAVES * q) * np];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) g += x[q];
         }
-        const float mm = b1 * m[p] + (1.f - b1) * g, vv = b2 * v[p] + (1.f - b2) * g * g;
-        m[p] = mm;
-        v[p] = vv;
-        par[p] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
+        for (; t < ntiles; t += MQE_WAVES) g += src[(size_t)t * np];
     }
+    part[w][lane] = g;
+    __syncthreads();
+    if (w != 0 || p >= np) return;
+    g = 0.f;
+#pragma unroll
+    for (int q = 0; q < MQE_WAVES; ++q) g += part[q][lane];
+    if (grad_out) {
+        grad_out[p] = g;
+        return;
+    }
+    const float mm = b1 * m[p] + (1.f - b1) * g, vv = b2 * v[p] + (1.f - b2) * g * g;
+    m[p] = mm;
+    v[p] = vv;
+    par[p] -= lr * (mm / c1) / (sqrtf(vv / c2) + eps);
 }
 
 // Column mean and standard deviation of an n x dim row-major array (one
@@ -332,8 +357,8 @@ int mlp_fit_device(mqe_mlp *m, const float *dX, const float *dY, long n, int epo
             ++m->adam_t;
             const float c1 = 1.f - powf(b1, (float)m->adam_t), c2 = 1.f - powf(b2, (float)m->adam_t);
             const int tiles = (int)((nb + mlp::TS - 1) / mlp::TS);
-            hipLaunchKernelGGL(mlp::adam_kernel, dim3((unsigned)std::min<long>((m->np + 255) / 256, 1024)),
-                               dim3(256), 0, s, m->d_par, m->d_m, m->d_v, m->d_gpart, tiles, m->np, (float)lr, b1,
+            hipLaunchKernelGGL(mlp::adam_kernel, dim3((unsigned)((m->np + mlp::SUM_P - 1) / mlp::SUM_P)),
+                               dim3(MQE_NT), 0, s, m->d_par, m->d_m, m->d_v, m->d_gpart, tiles, m->np, (float)lr, b1,
                                b2, eps, c1, c2, (float *)nullptr);
             MCHK(hipGetLastError());
         }
@@ -483,7 +508,7 @@ int mqe_mlp_loss_grad(mqe_mlp *m, int n, const float *X, const float *Y, double 
     if (r) return r;
     const int tiles = (int)((n + mlp::TS - 1) / mlp::TS);
     // grad_out mode of the Adam kernel: the summed gradient, no update
-    hipLaunchKernelGGL(mlp::adam_kernel, dim3((unsigned)std::min<long>((m->np + 255) / 256, 1024)), dim3(256), 0,
+    hipLaunchKernelGGL(mlp::adam_kernel, dim3((unsigned)((m->np + mlp::SUM_P - 1) / mlp::SUM_P)), dim3(MQE_NT), 0,
                        m->stream, m->d_par, m->d_m, m->d_v, m->d_gpart, tiles, m->np, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f,
                        m->d_grad);
     MCHK(hipGetLastError());
