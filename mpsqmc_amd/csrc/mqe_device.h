@@ -931,79 +931,94 @@ __device__ __forceinline__ double lanes_sum(double v) {
     return v;
 }
 
+// 1 / sqrt(x) and 1 / x of a positive normal x to within rounding: the hardware's
+// approximations (about 1e-7) with one third-order correction
+__device__ __forceinline__ double rsqrt_d(double x) {
+    const double r = __builtin_amdgcn_rsq(x), e = fma(-x * r, r, 1.0);
+    return fma(r * e, fma(0.375, e, 0.5), r);
+}
+__device__ __forceinline__ double recip_d(double x) {
+    const double r = __builtin_amdgcn_rcp(x), e = fma(-x, r, 1.0);
+    return fma(r * e, 1.0 + e, r);
+}
+
 // ---------------------------------------------------------------------------
 // The same factorisation with every column in registers: LPC lanes own a column
-// (lane ln its rows ln + LPC t, t < NE), so m <= LPC NE and n <= 256 / LPC; only
-// the reflectors (V, ld m, in LDS) and tau pass through LDS.  The group of column
-// j + 1 forms its reflector as soon as it has applied reflector j: one barrier
-// per column.  load(r, c): element of A (called once per element, before the
-// first barrier); put_r(r, c, x): R(r, c) for r <= c, after the last barrier
-// (V may be overwritten there if want_q is false); want_q: put_q(r, c, x) gets
-// Q, after a barrier past the last read of V.  Ends without a barrier.
-// What bounds it: the chain of one column (LDS read, dot product, group sum,
-// norm, root and division, LDS write, barrier), which nothing overlaps within a
-// walker; columns in LDS or memory put two to three more loads on that chain.
+// (lane ln its rows ln + LPC t, t < NE), so m <= LPC NE and n <= threads / LPC.
+// Column j goes to LDS (V, ld LPC NE, n columns) as soon as reflector j - 1 is
+// applied to it, unscaled, and every group forms the reflector from it while it
+// applies it: v = (a_jj + sign(a_jj) |a|, a_j+1.., a_m), tau = 1 / (|a| (|a| +
+// |a_jj|)), so the norm, root and reciprocal need no exchange of their own and a
+// column costs one barrier.  tau: n doubles in LDS.
+// load(r, c): element of A (called once per element, before the first barrier);
+// put_r(r, c, x): R(r, c) for r <= c, after the last barrier (V may be
+// overwritten there if want_q is false); want_q: put_q(r, c, x) gets Q, after a
+// barrier past the last read of V.  Ends without a barrier.
+// What bounds it: the chain of one column (LDS read, dot products, group sums,
+// root and reciprocal, update, LDS write, barrier), which nothing overlaps within
+// a walker.  So rows past m are zeros instead of bounds checks, groups that are
+// done run along with a zero factor, and there is no division on the chain: with
+// the owner of a column forming its reflector first, and a branch per element,
+// one sweep over the 31 inner sites of a D = 32 chain added 1258 us to a step,
+// now 681 us.
 // ---------------------------------------------------------------------------
 template <int LPC, int NE, class Load, class PutR, class PutQ>
 __device__ __forceinline__ void qr_regs(int m, int n, double *V, double *tau, bool want_q, Load load, PutR put_r,
                                         PutQ put_q) {
+    constexpr int LDV = LPC * NE;
     const int g = threadIdx.x / LPC, ln = threadIdx.x % LPC;
-    double a[NE];
+    const int glast = __builtin_amdgcn_readfirstlane((int)(threadIdx.x | 63) / LPC);  // the wave's last column
+    double a[NE], x[NE];
 #pragma unroll
     for (int t = 0; t < NE; ++t) {
         const int r = ln + LPC * t;
         a[t] = r < m && g < n ? load(r, g) : 0.0;
+        x[t] = 0.0;
     }
     __syncthreads();  // V may overlay what load() reads
-    auto reflect = [&](int j) {
-        double ss = 0.0, alpha = 0.0;
+    double *vg = V + LDV * g + ln;
+    if (g == 0) {
 #pragma unroll
-        for (int t = 0; t < NE; ++t) {
-            const int r = ln + LPC * t;
-            if (r > j) ss += a[t] * a[t];
-            if (r == j) alpha = a[t];
-        }
-        ss = lanes_sum<LPC>(ss);
-        alpha = lanes_sum<LPC>(alpha);
-        double tj = 0.0, sc = 0.0, beta = alpha;
-        if (ss != 0.0) {
-            beta = -copysign(sqrt(alpha * alpha + ss), alpha);
-            tj = (beta - alpha) / beta;
-            sc = 1.0 / (alpha - beta);
-        }
-        double *vj = V + (size_t)m * j;
-#pragma unroll
-        for (int t = 0; t < NE; ++t) {
-            const int r = ln + LPC * t;
-            if (r > j && r < m) {
-                a[t] *= sc;
-                vj[r] = a[t];
-            }
-            if (r == j) a[t] = beta;
-        }
-        if (ln == 0) tau[j] = tj;
-    };
-    // x <- H_j x, x in the rows of this lane
-    auto apply = [&](int j, double tj, double (&x)[NE]) {
-        const double *vj = V + (size_t)m * j;
-        double vr[NE], s = 0.0;
-#pragma unroll
-        for (int t = 0; t < NE; ++t) {
-            const int r = ln + LPC * t;
-            vr[t] = r > j && r < m ? vj[r] : (r == j ? 1.0 : 0.0);
-        }
-#pragma unroll
-        for (int t = 0; t < NE; ++t) s += vr[t] * x[t];
-        s = tj * lanes_sum<LPC>(s);
-#pragma unroll
-        for (int t = 0; t < NE; ++t) x[t] -= s * vr[t];
-    };
-    if (g == 0) reflect(0);
+        for (int t = 0; t < NE; ++t) vg[LPC * t] = a[t];
+    }
     __syncthreads();
     for (int j = 0; j < n; ++j) {
-        if (g > j && g < n) {
-            apply(j, tau[j], a);
-            if (g == j + 1) reflect(j + 1);
+        if (g == j - 1) {  // v_{j-1} in its final form, for Q
+#pragma unroll
+            for (int t = 0; t < NE; ++t) vg[LPC * t] = x[t];
+        }
+        if (glast >= j) {
+            // the raw column j; the rows above j hold R already
+            const double *vj = V + LDV * j;
+            const double alpha = vj[j];
+            double ss = 0.0, s = 0.0, aj = 0.0;
+#pragma unroll
+            for (int t = 0; t < NE; ++t) x[t] = vj[ln + LPC * t];
+#pragma unroll
+            for (int t = 0; t < NE; ++t) {
+                const int r = ln + LPC * t;
+                x[t] = r > j ? x[t] : 0.0;
+                aj += r == j ? a[t] : 0.0;
+                ss += x[t] * x[t];
+                s += x[t] * a[t];
+            }
+            ss = lanes_sum<LPC>(ss);
+            s = lanes_sum<LPC>(s);
+            aj = lanes_sum<LPC>(aj);
+            const double n2 = fma(alpha, alpha, ss), nrm = n2 * rsqrt_d(n2), d = nrm + fabs(alpha);
+            const bool on = ss > 0.0 && n2 > 1e-290;  // (the squares of anything smaller are lost to underflow)
+            const double vjj = on ? copysign(d, alpha) : 1.0, tj = on ? recip_d(nrm * d) : 0.0;
+            const double f = g >= j ? tj * fma(vjj, aj, s) : 0.0;
+#pragma unroll
+            for (int t = 0; t < NE; ++t) {
+                x[t] = ln + LPC * t == j ? vjj : x[t];
+                a[t] = fma(-f, x[t], a[t]);
+            }
+            if (g == j) tau[j] = tj;
+            if (g == j + 1 && g < n) {
+#pragma unroll
+                for (int t = 0; t < NE; ++t) vg[LPC * t] = a[t];
+            }
         }
         __syncthreads();
     }
@@ -1015,12 +1030,36 @@ __device__ __forceinline__ void qr_regs(int m, int n, double *V, double *tau, bo
         }
     }
     if (!want_q) return;
+    if (g == n - 1) {
+#pragma unroll
+        for (int t = 0; t < NE; ++t) vg[LPC * t] = x[t];
+    }
+    __syncthreads();
     // Q column c = H_0 H_1 ... H_c e_c; the groups of a wave take the same
-    // reflector at the same time, so its LDS reads are broadcasts
+    // reflector at the same time, so its LDS reads are broadcasts, and the next
+    // reflector is read while the current one is applied
 #pragma unroll
     for (int t = 0; t < NE; ++t) a[t] = ln + LPC * t == g ? 1.0 : 0.0;
-    for (int k = min(n - 1, (int)((threadIdx.x | 63) / LPC)); k >= 0; --k)
-        if (k <= g) apply(k, tau[k], a);
+    const int k0 = min(n - 1, glast);
+    double tk = tau[k0];
+#pragma unroll
+    for (int t = 0; t < NE; ++t) x[t] = V[LDV * k0 + ln + LPC * t];
+    for (int k = k0; k >= 0; --k) {
+        const int kn = max(k - 1, 0);
+        double y[NE], s = 0.0;
+        const double tn = tau[kn];
+#pragma unroll
+        for (int t = 0; t < NE; ++t) y[t] = V[LDV * kn + ln + LPC * t];
+#pragma unroll
+        for (int t = 0; t < NE; ++t) s += x[t] * a[t];
+        s = k <= g ? tk * lanes_sum<LPC>(s) : 0.0;
+#pragma unroll
+        for (int t = 0; t < NE; ++t) {
+            a[t] = fma(-s, x[t], a[t]);
+            x[t] = y[t];
+        }
+        tk = tn;
+    }
     __syncthreads();
     if (g < n) {
 #pragma unroll
@@ -1031,8 +1070,10 @@ __device__ __forceinline__ void qr_regs(int m, int n, double *V, double *tau, bo
     }
 }
 
-// qr_regs with the split by size: 8 lanes a column up to 64 x 32, 4 lanes up to 128 x 64
+// qr_regs with the split by size: 8 lanes a column up to 64 x 32, 4 lanes up to
+// 128 x 64.  qr_doubles: LDS of V and tau for any matrix of at most 2 D x D.
 constexpr int QR_REGS_M = 128, QR_REGS_N = 64;
+__host__ __device__ constexpr long qr_doubles(int D) { return (D <= 32 ? 64L : 128L) * D + D; }
 template <class Load, class PutR, class PutQ>
 __device__ __forceinline__ void qr_in_regs(int m, int n, double *V, double *tau, bool want_q, Load load, PutR put_r,
                                            PutQ put_q) {

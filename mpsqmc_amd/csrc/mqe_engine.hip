@@ -259,7 +259,10 @@ __device__ __forceinline__ void compress_bond(const Pool &P, T *phi, int *wv, in
 }
 
 // Doubles of one of the two work matrices of compress_bond.
-__host__ __device__ inline long compress_block(int Dmax) { return (2L * Dmax + 1) * Dmax; }
+__host__ __device__ inline long compress_block(int Dmax) {
+    const long x = (2L * Dmax + 1) * Dmax, q = qr_doubles(Dmax) - Dmax;
+    return Dmax <= QR_REGS_N && q > x ? q : x;  // QR in registers: its reflectors overlay the matrix
+}
 // Largest bond whose two work matrices, singular values and their order fit the LDS (160 KB per CU).
 constexpr int COMPRESS_LDS_D = 64;
 
@@ -1208,9 +1211,9 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
     }
     if (!e->tile32) {
         // the general kernel runs two workgroups per CU (launch bounds); its LQ
-        // workspace (Dw tau, then up to 2 Dw x Dw matrix columns) goes to LDS, as
-        // much as 72 KB holds
-        const size_t need = std::min(sizeof(double) * ((size_t)2 * e->Dw * e->Dw + e->Dw), (size_t)72 * 1024);
+        // workspace (reflectors and their factors, or the trailing columns of a
+        // larger matrix) goes to LDS, as much as 72 KB holds
+        const size_t need = std::min(sizeof(double) * (size_t)qr_doubles(e->Dw), (size_t)72 * 1024);
         if (need >= sizeof(double) * (size_t)(e->Dw + 2 * e->Dw)) {
             e->gen_lds_bytes = need;
             CK(lds_attr_f32_chained(need));

@@ -555,9 +555,10 @@ __device__ __forceinline__ void lq_site(const Ctx<T, CH> &C, int k) {
     const int m = 2 * wn, n = wk;
     T *ph = C.site(k);
     T *LM = C.ts + C.sl.LM;
-    if (C.qlds && n <= m && m <= QR_REGS_M && n <= QR_REGS_N && (long)m * n + C.S->Dw <= C.qlds_doubles) {
+    if (C.qlds && n <= m && m <= QR_REGS_M && n <= QR_REGS_N &&
+        C.qlds_doubles >= (m <= 64 && n <= 32 ? 65L : 129L) * n) {
         qr_in_regs(
-            m, n, C.qlds + C.S->Dw, C.qlds, true, [&](int r, int c) { return (double)ph[c + (size_t)wk * r]; },
+            m, n, C.qlds + n, C.qlds, true, [&](int r, int c) { return (double)ph[c + (size_t)wk * r]; },
             [&](int r, int c, double x) {
                 LM[c + (size_t)n * r] = (T)x;
                 if (r != c) LM[r + (size_t)n * c] = T(0);

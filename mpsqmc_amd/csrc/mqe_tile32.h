@@ -232,125 +232,21 @@ struct W32 {
 // phi = Lmat Q with Q right-orthonormal.  Q overwrites the center blocks and
 // Lmat (lower triangular, w_k x w_k) goes to B_LM.  The transposed matrix
 // A = phi^T (m = 2 w_{k+1} <= 64 rows, n = w_k <= 32 columns) is factorised
-// with row index r = col + w_{k+1} s.  32 groups of 8 lanes: group g keeps
-// column g in registers (lane ln holds rows ln + 8t, t = 0..7); only the
-// reflector vectors and tau pass through LDS (V: 64 x 32 doubles, column j at
-// V + 64 j), one workgroup barrier per column.
+// with row index r = col + w_{k+1} s by 32 groups of 8 lanes, one column each.
 // ---------------------------------------------------------------------------
 
-__device__ void lq32(const W32 &C, int wk, int wn, float *center) {
-    const int m = 2 * wn, n = wk;
-    double *V = (double *)C.blk(B_N), *tau = V + 64 * 32;
-    const int tid = threadIdx.x, g = tid >> 3, ln = tid & 7;
-    // this group's column of A = phi^T
-    double a[8];
-#pragma unroll
-    for (int t = 0; t < 8; ++t) {
-        const int r = ln + 8 * t;
-        double v = 0.0;
-        if (r < m && g < n) {
-            const int s = r >= wn ? 1 : 0, col = r - s * wn;
-            v = (double)center[s * BLK + g + LD * col];
-        }
-        a[t] = v;
-    }
-    // Householder reflector of the own column j (rows j..m-1): v_j = 1 implied,
-    // v_i (i > j) written to V, beta kept in a (row j), tau to LDS.
-    auto reflect = [&](int j) {
-        double ss = 0.0, alpha = 0.0;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int r = ln + 8 * t;
-            if (r > j) ss += a[t] * a[t];
-            if (r == j) alpha = a[t];
-        }
-        ss = group8_sum(ss);
-        alpha = group8_sum(alpha);
-        double tj = 0.0, sc = 0.0, beta = alpha;
-        if (ss != 0.0) {
-            beta = -copysign(sqrt(alpha * alpha + ss), alpha);
-            tj = (beta - alpha) / beta;
-            sc = 1.0 / (alpha - beta);
-        }
-        double *vj = V + 64 * j;
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int r = ln + 8 * t;
-            if (r > j) {
-                if (tj != 0.0) a[t] *= sc;
-                vj[r] = (tj != 0.0) ? a[t] : 0.0;
-            }
-            if (r == j) a[t] = beta;
-        }
-        if (ln == 0) tau[j] = tj;
-    };
-    if (g == 0) reflect(0);
-    __syncthreads();
-    for (int j = 0; j < n; ++j) {
-        if (g > j && g < n) {
-            const double tj = tau[j];
-            if (tj != 0.0) {
-                const double *vj = V + 64 * j;
-                double vr[8];
-#pragma unroll
-                for (int t = 0; t < 8; ++t) {
-                    const int r = ln + 8 * t;
-                    vr[t] = (r > j && r < m) ? vj[r] : (r == j ? 1.0 : 0.0);
-                }
-                double s = 0.0;
-#pragma unroll
-                for (int t = 0; t < 8; ++t) s += vr[t] * a[t];
-                s = tj * group8_sum(s);
-#pragma unroll
-                for (int t = 0; t < 8; ++t) a[t] -= s * vr[t];
-            }
-            if (g == j + 1) reflect(j + 1);
-        }
-        __syncthreads();
-    }
-    // Lmat = R^T (lower): R(j, g) for j <= g is held in group g, row j
+__device__ __forceinline__ void lq32(const W32 &C, int wk, int wn, float *center) {
     float *LM = C.blk(B_LM);
-    for (int e = tid; e < BLK; e += MQE_NT) LM[e] = 0.f;
-    __syncthreads();
-    if (g < n) {
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int r = ln + 8 * t;
-            if (r <= g) LM[g + LD * r] = (float)a[t];  // Lmat(g, r) = R(r, g)
-        }
-    }
-    // Q column c = H_0 H_1 ... H_c e_c, group c; written transposed into the center
-    if (g < n) {
-        const int c = g;
-        double q[8];
-#pragma unroll
-        for (int t = 0; t < 8; ++t) q[t] = (ln + 8 * t == c) ? 1.0 : 0.0;
-        for (int k = c; k >= 0; --k) {
-            const double tk = tau[k];
-            if (tk == 0.0) continue;
-            const double *vk = V + 64 * k;
-            double vr[8];
-#pragma unroll
-            for (int t = 0; t < 8; ++t) {
-                const int r = ln + 8 * t;
-                vr[t] = (r > k && r < m) ? vk[r] : (r == k ? 1.0 : 0.0);
-            }
-            double s = 0.0;
-#pragma unroll
-            for (int t = 0; t < 8; ++t) s += vr[t] * q[t];
-            s = tk * group8_sum(s);
-#pragma unroll
-            for (int t = 0; t < 8; ++t) q[t] -= s * vr[t];
-        }
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int r = ln + 8 * t;
-            if (r < m) {
-                const int s = r >= wn ? 1 : 0, col = r - s * wn;
-                center[s * BLK + c + LD * col] = (float)q[t];
-            }
-        }
-    }
+    double *V = (double *)C.blk(B_N);
+    for (int e = threadIdx.x; e < BLK; e += MQE_NT) LM[e] = 0.f;
+    auto el = [&](int r, int c) -> float & {
+        const int s = r >= wn ? 1 : 0;
+        return center[s * BLK + c + LD * (r - s * wn)];
+    };
+    qr_regs<8, 8>(
+        2 * wn, wk, V, V + 64 * 32, true, [&](int r, int c) { return (double)el(r, c); },
+        [&](int r, int c, double x) { LM[c + LD * r] = (float)x; },  // Lmat = R^T
+        [&](int r, int c, double x) { el(r, c) = (float)x; });
     __syncthreads();
 }
 
