@@ -1230,6 +1230,10 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
     {
         std::vector<int> fill(csptr.begin(), csptr.end());
         for (int c = 0; c < nC; ++c) csidx[fill[second[c]]++] = c;
+        // by first site: the energy sweep picks partners up from left to right
+        for (int k = 0; k < L; ++k)
+            std::stable_sort(csidx.begin() + csptr[k], csidx.begin() + csptr[k + 1],
+                             [&](int a, int b) { return first[a] < first[b]; });
     }
     auto up = [&](void **dst, const void *src, size_t bytes) -> hipError_t {
         hipError_t r = hipMalloc(dst, std::max(bytes, (size_t)8));

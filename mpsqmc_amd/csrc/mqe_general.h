@@ -317,13 +317,27 @@ __device__ __forceinline__ double pair_energy3(const Ctx<T, CH> &C, int tb, int 
     return block_sum(acc, C.red);
 }
 
-// Mixed tensor for the pair (i, j) from L_i, sites i..j and R_{j+1}.
+// The four blocks G(s', s) of site `first` carried to the left of site `bond`
+// (contiguous channels at A, B is the other buffer); first < 0: none.
+template <typename T>
+struct Carried {
+    int first, bond;
+    T *A, *B;
+};
+
+// Mixed tensor for the pair (i, j) from L_i, sites i..j and R_{j+1}.  `more`: the
+// next coupling has the same first site and will take the channels on from bond
+// j (in a torus or a frustrated lattice a site has several partners to its right:
+// 85 instead of 248 carries in the 4x4 torus with diagonals; with the same for
+// the energy and uniform addresses a step of 48 walkers at D = 20 in FP64 went
+// from 7.6 to 3.25 ms).
 template <typename T, bool CH>
-__device__ __forceinline__ void pair_for_coupling(const Ctx<T, CH> &C, int i, int j, double *M) {
+__device__ __forceinline__ void pair_for_coupling(const Ctx<T, CH> &C, int i, int j, bool more, Carried<T> &cr,
+                                                  double *M) {
     const int tn = C.tv[i + 1], wn = C.wv[i + 1];
     const T *g[4];
     int gld;
-    if (j == i + 1) {
+    if (j == i + 1 && !more) {
         T *G = C.ts + C.sl.G;
         if constexpr (CH) {  // G and V in one barrier interval
             issue_V(C, j, issue_G(C, i, C.Lk(i), G, 2 * tn, tn, (long)wn * 2 * tn, 0));
@@ -339,19 +353,22 @@ __device__ __forceinline__ void pair_for_coupling(const Ctx<T, CH> &C, int i, in
         gld = 2 * tn;
     } else {
         // the four blocks as contiguous channels (ch = 2 s' + s), carried to bond j
-        T *A = C.ts + C.sl.GcA, *B = C.ts + C.sl.GcB;
-        if constexpr (CH) {  // G channels and V in one barrier interval
-            issue_V(C, j, compute_G_channels(C, i, A));
-            __syncthreads();
-        } else {
-            compute_G_channels(C, i, A);
+        int wq = 0;
+        if (cr.first != i || cr.bond > j) {
+            wq = compute_G_channels(C, i, cr.A);
+            cr.first = i;
+            cr.bond = i + 1;
         }
-        for (int k = i + 1; k < j; ++k) {
-            carry_channels(C, k, A, B);
-            T *t = A; A = B; B = t;
+        if constexpr (CH) {  // G channels and V in one barrier interval
+            issue_V(C, j, wq);
+            __syncthreads();
+        }
+        for (; cr.bond < j; ++cr.bond) {
+            carry_channels(C, cr.bond, cr.A, cr.B);
+            T *t = cr.A; cr.A = cr.B; cr.B = t;
         }
         const int tb = C.tv[j], wb = C.wv[j];
-        for (int ch = 0; ch < 4; ++ch) g[ch] = A + (size_t)ch * tb * wb;
+        for (int ch = 0; ch < 4; ++ch) g[ch] = cr.A + (size_t)ch * tb * wb;
         gld = tb;
         if constexpr (!CH) compute_V(C, j);
     }
@@ -681,11 +698,11 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
                 }
             }
             if constexpr (CH) {
-                // V, M_k and the nearest-neighbour G of bond k (the last coupling
-                // ending at k, if it is (k-1, k)) in one barrier interval
+                // V, M_k and the nearest-neighbour G of bond k (if (k-1, k) is the only
+                // coupling ending at k) in one barrier interval
                 const int wq = issue_M(C, k, issue_V(C, k, 0));
                 const int ql = S.cs_ptr[k + 1] - 1;
-                if (ql >= S.cs_ptr[k] && S.first[S.cs_idx[ql]] == k - 1) {
+                if (ql == S.cs_ptr[k] && S.first[S.cs_idx[ql]] == k - 1) {
                     const int tn = C.tv[k], wn = C.wv[k];
                     issue_G(C, k - 1, C.Lk(k - 1), C.ts + C.sl.G, 2 * tn, tn, (long)wn * 2 * tn, wq);
                     nn_ready = true;
@@ -705,51 +722,61 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
             }
             if constexpr (!CH) advance_M(C, k);
         }
-        for (int q = S.cs_ptr[k]; q < S.cs_ptr[k + 1]; ++q) {
-            const int c = S.cs_idx[q], i = S.first[c];
+        const int q0 = S.cs_ptr[k], nq = S.cs_ptr[k + 1] - q0;
+        if (nq == 1 && S.first[S.cs_idx[q0]] == k - 1) {
+            const int c = S.cs_idx[q0], i = k - 1;
             const int tn = C.tv[i + 1], wn = C.wv[i + 1];
             const T *g[4];
-            int gld;
-            if (i == k - 1) {
-                if (!nn_ready) compute_G(C, i, C.Lk(i));
-                const T *G = C.ts + C.sl.G;
-                for (int ch = 0; ch < 4; ++ch) {
-                    const int sp = ch >> 1, s = ch & 1;
-                    g[ch] = G + (size_t)sp * tn + (size_t)s * wn * 2 * tn;
-                }
-                gld = 2 * tn;
-            } else {
-                // long range: only S_i . S_k is needed, so the four channels G(s', s)
-                // are combined into the three operator channels S^z, S^+, S^- of
-                // site i (ch = 2 s' + s: S^z = (G(1,1) - G(0,0)) / 2, S^+ = G(1,0),
-                // S^- = G(0,1)) and three are carried instead of four
-                T *A = C.ts + C.sl.GcA, *B = C.ts + C.sl.GcB;
-                compute_G_channels(C, i, A);
-                if constexpr (CH) __syncthreads();
-                {
-                    const int nb = tn * wn;
-                    for (int e = threadIdx.x; e < nb; e += MQE_NT) {
-                        const T g00 = A[e], g01 = A[nb + e], g10 = A[2 * nb + e], g11 = A[3 * nb + e];
-                        A[e] = (T)0.5 * (g11 - g00);
-                        A[nb + e] = g10;
-                        A[2 * nb + e] = g01;
-                    }
-                    __syncthreads();
-                }
-                for (int kk = i + 1; kk < k; ++kk) {
-                    carry_channels(C, kk, A, B, 3);
-                    T *t = A; A = B; B = t;
-                }
-                const double e = pair_energy3(C, C.tv[k], C.wv[k], A, r_pending ? C.Rk(k) : nullptr);
-                r_pending = false;
-                etot += S.Jc[c] * e;
-                continue;
+            if (!nn_ready) compute_G(C, i, C.Lk(i));
+            const T *G = C.ts + C.sl.G;
+            for (int ch = 0; ch < 4; ++ch) {
+                const int sp = ch >> 1, s = ch & 1;
+                g[ch] = G + (size_t)sp * tn + (size_t)s * wn * 2 * tn;
             }
-            pair_tensor(C, C.tv[k], C.wv[k], g, gld, M, r_pending ? C.Rk(k) : nullptr);
-            r_pending = false;
+            pair_tensor(C, C.tv[k], C.wv[k], g, 2 * tn, M, r_pending ? C.Rk(k) : nullptr);
             double e = 0.0;
             for (int q2 = 0; q2 < 16; ++q2) e += S.SS[q2] * M[q2];
             etot += S.Jc[c] * e;
+        } else if (nq > 0) {
+            // only sum_i J_ik S_i . S_k is needed: the operator channels S^z, S^+, S^-
+            // of site i (ch = 2 s' + s: S^z = (G(1,1) - G(0,0)) / 2, S^+ = G(1,0),
+            // S^- = G(0,1)) times J_ik start at the leftmost partner of k, take in
+            // each further one on their way right, and meet V once at bond k
+            T *A = C.ts + C.sl.GcA, *B = C.ts + C.sl.GcB;
+            int bond = -1;
+            for (int q = q0; q <= q0 + nq; ++q) {
+                const int c = q < q0 + nq ? S.cs_idx[q] : 0, i = q < q0 + nq ? S.first[c] : k - 1;
+                const int tn = C.tv[i + 1], wn = C.wv[i + 1];
+                T *G = C.ts + C.sl.G;
+                if (q < q0 + nq) {
+                    if constexpr (CH) {
+                        issue_G(C, i, C.Lk(i), G, 2 * tn, tn, (long)wn * 2 * tn, 0);
+                        if (bond < 0 || bond > i) __syncthreads();
+                    } else {
+                        compute_G(C, i, C.Lk(i));
+                    }
+                }
+                const bool fresh = bond < 0;
+                for (int kk = fresh ? i + 1 : bond; kk <= i; ++kk) {
+                    carry_channels(C, kk, A, B, 3);
+                    T *t = A; A = B; B = t;
+                }
+                bond = i + 1;
+                if (q == q0 + nq) break;
+                const int nb = tn * wn;
+                const double J = S.Jc[c];
+                for (int e = threadIdx.x; e < nb; e += MQE_NT) {
+                    const int a = e % tn, be = e / tn;
+                    const size_t o = a + (size_t)2 * tn * be, os = (size_t)wn * 2 * tn;
+                    const T g00 = G[o], g01 = G[o + os], g10 = G[o + tn], g11 = G[o + tn + os];
+                    const double z = 0.5 * J * ((double)g11 - (double)g00), pl = J * g10, mi = J * g01;
+                    A[e] = (T)(fresh ? z : (double)A[e] + z);
+                    A[nb + e] = (T)(fresh ? pl : (double)A[nb + e] + pl);
+                    A[2 * nb + e] = (T)(fresh ? mi : (double)A[2 * nb + e] + mi);
+                }
+                __syncthreads();
+            }
+            etot += pair_energy3(C, C.tv[k], C.wv[k], A, r_pending ? C.Rk(k) : nullptr);
         }
         if (S.h != 0.0) {
             // <trial|S^z_k|phi> = sum_t sz[t] <L'_k, V(t,t)>, L'_k the current-gauge left env
@@ -942,8 +969,10 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
     // header), and the energy sweep takes the norm.  rv: right environments R_k are
     // valid for k >= rv.
     int rv = 1;
+    Carried<T> cr{-1, 0, C.ts + C.sl.GcA, C.ts + C.sl.GcB};
     for (int c = 0; c < S.nC; ++c) {
         const int i = S.first[c], j = S.second[c];
+        const bool more = S.nextfirst[c] == i;
         // the left environments up to L_i and the right ones down to R_{j+1}: two
         // independent chains (CH: one step of each per barrier interval)
         if constexpr (CH) {
@@ -960,7 +989,7 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
             }
             while (rv > j + 1) rebuild_R(C, --rv);
         }
-        pair_for_coupling(C, i, j, M);
+        pair_for_coupling(C, i, j, more, cr, M);
         const double *tS = S.tS + 4 * c, *tU = S.tU + 16 * c, *tVT = S.tVT + 16 * c;
         const double u = P.u ? P.u[(size_t)b * S.nC + c] : philox_uniform(P.seed, (uint32_t)b, (uint32_t)c, (uint32_t)ctl.step, 0u);
         double pdfnorm, fstar, Ux[4], Vx[4];
@@ -1036,6 +1065,13 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
                     v11 = (T)(alpha * Vx[3]);
             mix_pair(pi, bi, u00, u01, u10, u11);
             mix_pair(pj, bj, v00, v01, v10, v11);
+            if (more) {  // the carried channels with the new site i
+                const int nb = tv[j] * wv[j];
+                mix_pair(cr.A, nb, u00, u01, u10, u11);
+                mix_pair(cr.A + 2 * (size_t)nb, nb, u00, u01, u10, u11);
+            } else {
+                cr.first = -1;
+            }
             if (nn_move) {
                 const int tn = tv[i + 1], wn = wv[i + 1];
                 const T *G = C.ts + C.sl.G;
