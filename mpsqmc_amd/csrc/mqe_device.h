@@ -576,7 +576,7 @@ __device__ __forceinline__ int chain2(int wave0, int nu, int m1, int n1, int k1,
             v16f_c F0, F1;
 #pragma unroll
             for (int e = 0; e < 16; ++e) F0[e] = F1[e] = 0.f;
-            const auto rA = buf_rsrc(op.A), rB = buf_rsrc(op.B[f]);
+            const auto rA = buf_rsrc(op.A), rB = buf_rsrc(f == 0 ? op.B[0] : op.B[1]);
             auto slice = [&](int k0, bool tail) {
                 float a0[8], a1[8], bv[8];
                 const int kl = k0 + 8 * h;
@@ -618,7 +618,7 @@ __device__ __forceinline__ int chain2(int wave0, int nu, int m1, int n1, int k1,
 #pragma unroll
                     for (int e = 0; e < 16; ++e) D0[e] = D1[e] = 0.f;
                 }
-                const float *Cp = op.C[ND == 1 ? f : d];
+                const float *Cp = (ND == 1 ? f : d) == 0 ? op.C[0] : op.C[1];
                 const auto rC = buf_rsrc(Cp);
                 const bool vecC = TC && (m1 & 3) == 0 && (ldc & 3) == 0 && aligned16(Cp, Cp, 0, 0);
                 auto chunk = [&](int row, int t, float (&cv)[16]) {
@@ -651,7 +651,7 @@ __device__ __forceinline__ int chain2(int wave0, int nu, int m1, int n1, int k1,
                 if (f == NF - 1) {
                     // rows 8(e/4) + 4h + e%4 (+32) of column c0 + r; outside D the store is dropped
                     const int vd = c0 + r < n1 ? 4 * (ldd * (c0 + r) + 4 * h) : BUF_OOB;
-                    const auto rD = buf_rsrc(op.D[d]);
+                    const auto rD = buf_rsrc(d == 0 ? op.D[0] : op.D[1]);
                     if (do0) {
 #pragma unroll
                         for (int e = 0; e < 16; ++e) {
@@ -740,7 +740,7 @@ __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int 
             V4 F[4];
 #pragma unroll
             for (int t = 0; t < 4; ++t) F[t] = V4{0, 0, 0, 0};
-            const auto rA = buf_rsrc(op.A), rB = buf_rsrc(op.B[f]);
+            const auto rA = buf_rsrc(op.A), rB = buf_rsrc(f == 0 ? op.B[0] : op.B[1]);
             // the last, partial slice takes k = kf + 4q + g, so that a step wholly past k1 is left out
             auto slice = [&](int k0, bool tail) {
                 T a[4][4], bv[4];
@@ -775,7 +775,7 @@ __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int 
 #pragma nounroll
             for (int d = 0; d < ND; ++d) {
                 asm volatile("" : "+v"(c), "+v"(g));
-                const T *Cp = op.C[ND == 1 ? f : d];
+                const T *Cp = (ND == 1 ? f : d) == 0 ? op.C[0] : op.C[1];
                 const auto rC = buf_rsrc(Cp);
                 const bool vecC = TC && SZ == 4 && (m1 & 3) == 0 && (ldc & 3) == 0 && (((uintptr_t)Cp) & 15u) == 0;
                 if (ND == 2 || f == 0) {
@@ -814,7 +814,7 @@ __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int 
                 if (f == NF - 1) {
                     // row 16 qd + row(g, e) of column c0 + c; outside D the store is dropped
                     const int vd = c0 + c < n1 ? SZ * (ldd * (c0 + c) + CT::ROW_G * g) : BUF_OOB;
-                    const auto rD = buf_rsrc(op.D[d]);
+                    const auto rD = buf_rsrc(d == 0 ? op.D[0] : op.D[1]);
 #pragma unroll
                     for (int qd = 0; qd < 4; ++qd) {
                         if (qd < q0 || qd >= q1) continue;

@@ -8,6 +8,21 @@
 
 namespace mqe {
 
+// Wave-uniform values.  Bond dimensions, site numbers and the tensors' addresses
+// are the same in every lane of a workgroup, but the compiler cannot know it of
+// values that come from LDS or memory: held in vector registers they made every
+// loop bound a lane mask, every address 64-bit vector arithmetic and every buffer
+// resource a loop over the lanes' values.
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ long uni(long x) {
+    const unsigned lo = (unsigned)uni((int)(unsigned)x), hi = (unsigned)uni((int)(unsigned)((unsigned long)x >> 32));
+    return (long)(((unsigned long)hi << 32) | lo);
+}
+struct UniDims {  // bond dimensions in LDS, read as uniform values
+    const int *p;
+    __device__ __forceinline__ int operator[](int k) const { return uni(p[k]); }
+};
+
 // ---------------------------------------------------------------------------
 // per-walker context
 // ---------------------------------------------------------------------------
@@ -19,7 +34,7 @@ struct Ctx {
     const T *trial;
     T *phi, *Lenv, *Renv;
     const long *woff, *eoff, *moff;
-    const int *tv, *wv;  // LDS copies of bond dims
+    UniDims tv, wv;      // LDS copies of bond dims
     ScratchLayout sl;
     T *ts;               // T scratch
     double *ds;          // double scratch
@@ -30,20 +45,20 @@ struct Ctx {
 
     const float *trialT; // FP32: the trial with every T_k[s] transposed (t_{k+1} x t_k), or nullptr
 
-    __device__ T *site(int k) const { return phi + woff[k]; }
-    __device__ const T *tsite(int k) const { return trial + S->toff[k]; }
+    __device__ T *site(int k) const { return phi + uni(woff[k]); }
+    __device__ const T *tsite(int k) const { return trial + uni(S->toff[k]); }
     // site k of the trial as the second operand of a product T_k[s] F: FP32 takes
     // the transposed copy (four values along the inner index per load), FP64 the
     // plain one (its inner index is strided over the lanes)
     static constexpr bool TRT = sizeof(T) == sizeof(float);
     __device__ const T *tsiteR(int k) const {
-        if constexpr (TRT) return trialT + S->toff[k];
+        if constexpr (TRT) return trialT + uni(S->toff[k]);
         else return tsite(k);
     }
 
-    __device__ T *Lk(int k) const { return Lenv + eoff[k]; }
-    __device__ T *Rk(int k) const { return Renv + eoff[k]; }
-    __device__ T *Mk(int k) const { return Renv + moff[k]; }  // right norm environment (w_k x w_k)
+    __device__ T *Lk(int k) const { return Lenv + uni(eoff[k]); }
+    __device__ T *Rk(int k) const { return Renv + uni(eoff[k]); }
+    __device__ T *Mk(int k) const { return Renv + uni(moff[k]); }  // right norm environment (w_k x w_k)
 };
 
 // Chained-product issue functions (CH instance only): they start their items at
@@ -701,8 +716,8 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
                 // V, M_k and the nearest-neighbour G of bond k (if (k-1, k) is the only
                 // coupling ending at k) in one barrier interval
                 const int wq = issue_M(C, k, issue_V(C, k, 0));
-                const int ql = S.cs_ptr[k + 1] - 1;
-                if (ql == S.cs_ptr[k] && S.first[S.cs_idx[ql]] == k - 1) {
+                const int ql = uni(S.cs_ptr[k + 1]) - 1;
+                if (ql == uni(S.cs_ptr[k]) && uni(S.first[S.cs_idx[ql]]) == k - 1) {
                     const int tn = C.tv[k], wn = C.wv[k];
                     issue_G(C, k - 1, C.Lk(k - 1), C.ts + C.sl.G, 2 * tn, tn, (long)wn * 2 * tn, wq);
                     nn_ready = true;
@@ -711,7 +726,7 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
             } else {
                 compute_V(C, k);
             }
-            if (S.cs_ptr[k + 1] > S.cs_ptr[k]) {
+            if (uni(S.cs_ptr[k + 1]) > uni(S.cs_ptr[k])) {
                 r_pending = true;  // R_k from the first pair tensor of the site
             } else {
                 const int tk = C.tv[k], wk = C.wv[k];
@@ -722,8 +737,8 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
             }
             if constexpr (!CH) advance_M(C, k);
         }
-        const int q0 = S.cs_ptr[k], nq = S.cs_ptr[k + 1] - q0;
-        if (nq == 1 && S.first[S.cs_idx[q0]] == k - 1) {
+        const int q0 = uni(S.cs_ptr[k]), nq = uni(S.cs_ptr[k + 1]) - q0;
+        if (nq == 1 && uni(S.first[S.cs_idx[q0]]) == k - 1) {
             const int c = S.cs_idx[q0], i = k - 1;
             const int tn = C.tv[i + 1], wn = C.wv[i + 1];
             const T *g[4];
@@ -745,7 +760,7 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
             T *A = C.ts + C.sl.GcA, *B = C.ts + C.sl.GcB;
             int bond = -1;
             for (int q = q0; q <= q0 + nq; ++q) {
-                const int c = q < q0 + nq ? S.cs_idx[q] : 0, i = q < q0 + nq ? S.first[c] : k - 1;
+                const int c = q < q0 + nq ? uni(S.cs_idx[q]) : 0, i = q < q0 + nq ? uni(S.first[c]) : k - 1;
                 const int tn = C.tv[i + 1], wn = C.wv[i + 1];
                 T *G = C.ts + C.sl.G;
                 if (q < q0 + nq) {
@@ -906,8 +921,8 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
     const int n = *P.n;
     if ((int)blockIdx.x >= n) return;
     if (*P.status & 4) return;  // the population overflowed: keep the state as it was
-    const int b = P.list ? P.list[blockIdx.x] : (int)blockIdx.x;  // population position
-    const int slot = P.order[b];
+    const int b = uni(P.list ? P.list[blockIdx.x] : (int)blockIdx.x);  // population position
+    const int slot = uni(P.order[b]);
     const Ctl ctl = *P.ctl;
     const int L = S.L;
 
@@ -929,7 +944,7 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
     __syncthreads();
 
     Ctx<T, CH> C;
-    C.tile = sh_tile;
+    C.tile = uni(sh_tile);
     C.S = &S;
     C.trial = trial;
     C.trialT = S.trialT;
@@ -939,8 +954,8 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
     C.woff = P.woff;
     C.eoff = P.eoff;
     C.moff = P.moff;
-    C.tv = tv;
-    C.wv = wv;
+    C.tv = UniDims{tv};
+    C.wv = UniDims{wv};
     C.sl = scratch_layout(S.Dt, S.Dw, S.Ng);
     char *base = P.scratch + (size_t)b * P.scratch_bytes;
     C.ts = (T *)base;
@@ -971,8 +986,8 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
     int rv = 1;
     Carried<T> cr{-1, 0, C.ts + C.sl.GcA, C.ts + C.sl.GcB};
     for (int c = 0; c < S.nC; ++c) {
-        const int i = S.first[c], j = S.second[c];
-        const bool more = S.nextfirst[c] == i;
+        const int i = uni(S.first[c]), j = uni(S.second[c]), inext = uni(S.nextfirst[c]);
+        const bool more = inext == i;
         // the left environments up to L_i and the right ones down to R_{j+1}: two
         // independent chains (CH: one step of each per barrier interval)
         if constexpr (CH) {
@@ -1056,24 +1071,24 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
         // for nearest neighbours whose next coupling starts right of i, the left
         // boundary moves to j: L_{i+1} = sum_{s,s0} Ux[s,s0] G(s, s0).  One pass.
         const double alpha = O / (4.0 * fstar);
-        const bool nn_move = j == i + 1 && S.nextfirst[c] > i;
+        const bool nn_move = j == i + 1 && inext > i;
         {
             T *pi = C.site(i), *pj = C.site(j);
-            const int bi = wv[i] * wv[i + 1], bj = wv[j] * wv[j + 1];
+            const int bi = C.wv[i] * C.wv[i + 1], bj = C.wv[j] * C.wv[j + 1];
             const T u00 = (T)Ux[0], u10 = (T)Ux[1], u01 = (T)Ux[2], u11 = (T)Ux[3];
             const T v00 = (T)(alpha * Vx[0]), v10 = (T)(alpha * Vx[1]), v01 = (T)(alpha * Vx[2]),
                     v11 = (T)(alpha * Vx[3]);
             mix_pair(pi, bi, u00, u01, u10, u11);
             mix_pair(pj, bj, v00, v01, v10, v11);
             if (more) {  // the carried channels with the new site i
-                const int nb = tv[j] * wv[j];
+                const int nb = C.tv[j] * C.wv[j];
                 mix_pair(cr.A, nb, u00, u01, u10, u11);
                 mix_pair(cr.A + 2 * (size_t)nb, nb, u00, u01, u10, u11);
             } else {
                 cr.first = -1;
             }
             if (nn_move) {
-                const int tn = tv[i + 1], wn = wv[i + 1];
+                const int tn = C.tv[i + 1], wn = C.wv[i + 1];
                 const T *G = C.ts + C.sl.G;
                 T *Ln = C.Lk(i + 1);
                 for (int e = threadIdx.x; e < tn * wn; e += MQE_NT) {
