@@ -366,7 +366,7 @@ __device__ int rscan_excl(int v, int *out_excl, int *sh) {
 }
 
 struct Book {
-    const int *n;
+    int *n;
     int *order, *order2;
     double *w, *O, *eh, *EL;
     double *sums;     // [0] sum w  [1] scaling  [2] E_T  [3] E_P  [4] Omega  [5] N
@@ -383,14 +383,9 @@ __global__ void set_ctl_kernel(Ctl *ctl, Ctl v) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *ctl = v;
 }
 
-// start of a captured step: next step number and propagation
-__global__ void advance_ctl_kernel(Ctl *ctl) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        ctl->step += 1;
-        ctl->pstep += 1;
-        ctl->pc += 1;
-    }
-}
+// what launch_list_kernel does with the control block first: leave it, set it
+// (an eager step), or advance it to the next step and propagation (a captured step)
+enum : int { CTL_KEEP = 0, CTL_SET = 1, CTL_ADVANCE = 2 };
 
 // Population positions in launch order, most work first: the walkers that
 // re-orthonormalise in this propagation (several times the work of a light
@@ -398,18 +393,24 @@ __global__ void advance_ctl_kernel(Ctl *ctl) {
 // population order.  Heavy walkers start in the first round of resident
 // workgroups instead of extending the last one.  key: scratch, one int per position.
 __global__ __launch_bounds__(RED_NT) void launch_list_kernel(const int *n_ptr, const int *order, const int *wvd,
-                                                             const int *since, int L, const Ctl *ctl, int *key,
-                                                             int *list) {
+                                                             const int *since, int L, Ctl *ctl, int ctl_mode, Ctl v,
+                                                             int *key, int *list) {
     __shared__ int cnt[16], base[16], carry[16];
     __shared__ int wcnt[RED_NT / 64][16];
     const int n = *n_ptr;
-    const Ctl c = *ctl;
+    Ctl c = ctl_mode == CTL_SET ? v : *ctl;
+    if (ctl_mode == CTL_ADVANCE) {
+        c.step += 1;
+        c.pstep += 1;
+        c.pc += 1;
+    }
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
     if (threadIdx.x < 16) {
         cnt[threadIdx.x] = 0;
         carry[threadIdx.x] = 0;
     }
-    __syncthreads();
+    __syncthreads();  // every thread has read the control block
+    if (ctl_mode != CTL_KEEP && threadIdx.x == 0) *ctl = c;
     for (int b = threadIdx.x; b < n; b += RED_NT) {
         const int slot = order[b];
         const int *wv = wvd + (size_t)slot * (L + 1);
@@ -458,9 +459,12 @@ __global__ __launch_bounds__(RED_NT) void launch_list_kernel(const int *n_ptr, c
     }
 }
 
+// The bookkeeping of a step (weight sum, energies, population control) is a few
+// latencies of one workgroup each: a step of its own takes them in one launch
+// (step_kernel), the separate kernels serve the calls of the single parts.
+
 // sum of weights; if device_scaling also scaling and E_T (MPSQMC2.cpp:480-484)
-__global__ __launch_bounds__(RED_NT) void sumw_kernel(Book B) {
-    __shared__ double sh[RED_NT / 64];
+__device__ __forceinline__ void sum_weights(const Book &B, double *sh) {
     const int n = *B.n;
     double s = 0.0;
     for (int b = threadIdx.x; b < n; b += RED_NT) s += B.w[B.order[b]];
@@ -474,11 +478,15 @@ __global__ __launch_bounds__(RED_NT) void sumw_kernel(Book B) {
         B.sums[5] = n;
     }
 }
+__global__ __launch_bounds__(RED_NT) void sumw_kernel(Book B) {
+    __shared__ double sh[RED_NT / 64];
+    sum_weights(B, sh);
+}
 
 // EnergyFunctionAndHistory (MPSQMC2.cpp:688-747).  from_ctl: step number from
 // the control block and a trace row for it (a step of mqe_step / mqe_run).
-__global__ __launch_bounds__(RED_NT) void energy_kernel(Book B, int step, int dofluct, int trace_row, int from_ctl) {
-    __shared__ double sh[RED_NT / 64];
+__device__ __forceinline__ void energies(const Book &B, int step, int dofluct, int trace_row, int from_ctl,
+                                         double *sh) {
     const int n = *B.n;
     if (from_ctl) {
         step = B.ctl->step;
@@ -511,12 +519,15 @@ __global__ __launch_bounds__(RED_NT) void energy_kernel(Book B, int step, int do
         }
     }
 }
+__global__ __launch_bounds__(RED_NT) void energy_kernel(Book B, int step, int dofluct, int trace_row, int from_ctl) {
+    __shared__ double sh[RED_NT / 64];
+    energies(B, step, dofluct, trace_row, from_ctl, sh);
+}
 
 // SeparatePopulationControl (MPSQMC2.cpp:613-686): copy counts, new order,
 // slot assignment for the extra copies.  scaling from host (>0) or B.sums[1].
-__global__ __launch_bounds__(RED_NT) void popcontrol_kernel(Book B, double host_scaling, const double *u, int nu,
-                                                            unsigned long long seed) {
-    __shared__ int shi[RED_NT / 64];
+__device__ __forceinline__ void control_population(const Book &B, double host_scaling, const double *u, int nu,
+                                                   unsigned long long seed, int *shi) {
     __shared__ int carry_draw, carry_pos, carry_extra, carry_free;
     const int n = *B.n;
     if (*B.status & 4) {  // an earlier overflow: leave the population as it is
@@ -606,15 +617,34 @@ __global__ __launch_bounds__(RED_NT) void popcontrol_kernel(Book B, double host_
     }
     if (threadIdx.x == 0) *B.n_extra = carry_extra;
 }
+__global__ __launch_bounds__(RED_NT) void popcontrol_kernel(Book B, double host_scaling, const double *u, int nu,
+                                                            unsigned long long seed) {
+    __shared__ int shi[RED_NT / 64];
+    control_population(B, host_scaling, u, nu, seed, shi);
+}
 
-// Copy walker data for the extra copies; then install the new order.  The
+__global__ __launch_bounds__(RED_NT) void step_kernel(Book B, unsigned long long seed) {
+    __shared__ double sh[RED_NT / 64];
+    __shared__ int shi[RED_NT / 64];
+    sum_weights(B, sh);
+    energies(B, 0, 1, -1, 1, sh);
+    __syncthreads();  // the sums are written, the weights read
+    control_population(B, -1.0, nullptr, 0, seed, shi);
+}
+
+// Copy walker data for the extra copies and install the new order and number
+// (neither is read here).  The
 // bulk (walker tensors and right environments of every copy) is spread over
 // the whole grid in 16-byte chunks where the layout allows it, so the copies
 // run at memory bandwidth instead of one workgroup per copy.
 template <typename T>
 __global__ __launch_bounds__(MQE_NT) void copy_walkers_kernel(Book B, Pool P, int L) {
-    const int ne = *B.n_extra;
+    const int ne = *B.n_extra, total = *B.n_new;
     const long gid = (long)blockIdx.x * MQE_NT + threadIdx.x, gsz = (long)gridDim.x * MQE_NT;
+    if (total <= B.cap) {
+        for (long b = gid; b < total; b += gsz) B.order[b] = B.order2[b];
+        if (gid == 0) *B.n = total;
+    }
     for (long e = gid; e < ne; e += gsz) {  // scalars, bond dims, bond energies
         const int src = B.copy_src[e], dst = B.copy_dst[e];
         P.w[dst] = P.w[src];
@@ -690,19 +720,6 @@ __global__ void advance_samples_kernel(const int *n, int nC, long *nsamp, long m
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         const long add = (long)(*n) * nC;
         if (*nsamp + add <= maxsamp) *nsamp += add;
-    }
-}
-
-__global__ void install_order_kernel(Book B) {
-    const int total = *B.n_new;
-    if (total > B.cap) return;
-    for (int b = blockIdx.x * blockDim.x + threadIdx.x; b < total; b += gridDim.x * blockDim.x) B.order[b] = B.order2[b];
-}
-
-__global__ void set_n_kernel(Book B, int *n) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        const int t = *B.n_new;
-        if (t <= B.cap) *n = t;
     }
 }
 
@@ -857,11 +874,14 @@ static Book make_book(mqe_engine *e) {
     return B;
 }
 
+static void fill_ctl(mqe_engine *e) {
+    e->ctl_host.canon_every = e->canon_every;
+    e->ctl_host.trace_cap = e->trace_cap;
+}
 // Copy a control block value to the device with a kernel (no memset or copy
 // node, so the same call may sit in front of a graph replay).
 static int push_ctl(mqe_engine *e) {
-    e->ctl_host.canon_every = e->canon_every;
-    e->ctl_host.trace_cap = e->trace_cap;
+    fill_ctl(e);
     hipLaunchKernelGGL(set_ctl_kernel, dim3(1), dim3(64), 0, e->stream, e->d_ctl, e->ctl_host);
     HIPCHK(hipGetLastError());
     return MQE_OK;
@@ -870,13 +890,13 @@ static int push_ctl(mqe_engine *e) {
 // F_PREP: canonical form and local energies of the loaded walkers.  F_PROP: one
 // propagation with the step words and phase of the control block, walkers in
 // the launch order of launch_list_kernel.
-static int launch_walker_any(mqe_engine *e, const double *u, int flags) {
+static int launch_walker_any(mqe_engine *e, const double *u, int flags, int ctl_mode = CTL_KEEP) {
     Pool P = make_pool(e, u);
     const bool prop = (flags & F_PROP) != 0;
     if (prop) {
         ++e->prop_count;
         hipLaunchKernelGGL(launch_list_kernel, dim3(1), dim3(RED_NT), 0, e->stream, e->d_n, e->d_order, e->d_wvd,
-                           e->d_since, e->L, e->d_ctl, e->d_key, e->d_list);
+                           e->d_since, e->L, e->d_ctl, ctl_mode, e->ctl_host, e->d_key, e->d_list);
         HIPCHK(hipGetLastError());
         P.list = e->d_list;
     }
@@ -960,19 +980,19 @@ static void launch_copy(mqe_engine *e) {
     hipLaunchKernelGGL(copy_walkers_kernel<T>, dim3(2048), dim3(MQE_NT), 0, e->stream, B, P, e->L);
 }
 
+static int launch_copy_any(mqe_engine *e) {
+    if (e->fp32) launch_copy<float>(e);
+    else launch_copy<double>(e);
+    HIPCHK(hipGetLastError());
+    return MQE_OK;
+}
+
 // population control with the step word of the control block
 static int enqueue_popcontrol(mqe_engine *e, double scaling, const double *du, int nu) {
     Book B = make_book(e);
     hipLaunchKernelGGL(popcontrol_kernel, dim3(1), dim3(RED_NT), 0, e->stream, B, scaling, du, nu, e->p.seed);
     HIPCHK(hipGetLastError());
-    if (e->fp32) launch_copy<float>(e);
-    else launch_copy<double>(e);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(install_order_kernel, dim3(16), dim3(256), 0, e->stream, B);
-    HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(set_n_kernel, dim3(1), dim3(64), 0, e->stream, B, e->d_n);
-    HIPCHK(hipGetLastError());
-    return MQE_OK;
+    return launch_copy_any(e);
 }
 
 static bool tune_cache_read(const mqe_engine *e, int *tiles);
@@ -1545,18 +1565,19 @@ int mqe_population_control(mqe_engine *e, double scaling, const double *uniforms
     return MQE_OK;
 }
 
-// One Walk step.  Eager: the control block is set to this step; in a graph
-// capture (captured = true) a kernel advances it instead, so the captured
-// launches carry no step-dependent argument.
+// One Walk step in four launches: the launch list (which also sets the control
+// block to this step), the walkers, the bookkeeping, the copies (which also
+// install the new order).  In a graph capture (captured = true) the control block
+// is advanced instead, so the captured launches carry no step-dependent argument.
+// Nine launches (the control block, the three parts of the bookkeeping, the order
+// and the number by themselves) made a step of 64 walkers of 10 sites at D = 8
+// (none of them canonical) 73 us, four 64 us.
 static int enqueue_step(mqe_engine *e, int step, bool captured) {
-    if (captured) {
-        hipLaunchKernelGGL(advance_ctl_kernel, dim3(1), dim3(64), 0, e->stream, e->d_ctl);
-        HIPCHK(hipGetLastError());
-    } else {
+    if (!captured) {
         e->ctl_host.step = e->ctl_host.pstep = step;
         e->ctl_host.pc = e->prop_count;
         e->prop_draws = e->pop_draws = step;
-        ECHK(push_ctl(e));
+        fill_ctl(e);
     }
     const bool timed = e->timing && !captured;
     if (timed) {
@@ -1569,18 +1590,15 @@ static int enqueue_step(mqe_engine *e, int step, bool captured) {
         }
         HIPCHK(hipEventRecord(e->tev[e->tev_used], e->stream));
     }
-    ECHK(launch_walker_any(e, nullptr, F_PROP));
+    ECHK(launch_walker_any(e, nullptr, F_PROP, captured ? CTL_ADVANCE : CTL_SET));
     if (timed) {
         HIPCHK(hipEventRecord(e->tev[e->tev_used + 1], e->stream));
         e->tev_used += 2;
     }
     Book B = make_book(e);
-    hipLaunchKernelGGL(sumw_kernel, dim3(1), dim3(RED_NT), 0, e->stream, B);
+    hipLaunchKernelGGL(step_kernel, dim3(1), dim3(RED_NT), 0, e->stream, B, e->p.seed);
     HIPCHK(hipGetLastError());
-    hipLaunchKernelGGL(energy_kernel, dim3(1), dim3(RED_NT), 0, e->stream, B, step, 1, -1, 1);
-    HIPCHK(hipGetLastError());
-    ECHK(enqueue_popcontrol(e, -1.0, nullptr, 0));
-    return MQE_OK;
+    return launch_copy_any(e);
 }
 
 int mqe_step(mqe_engine *e, int step) {
