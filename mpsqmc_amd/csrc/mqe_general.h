@@ -713,11 +713,11 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
                 }
             }
             if constexpr (CH) {
-                // V, M_k and the nearest-neighbour G of bond k (if (k-1, k) is the only
-                // coupling ending at k) in one barrier interval
+                // V, M_k and the nearest-neighbour G of bond k (the last coupling
+                // ending at k, if it is (k-1, k)) in one barrier interval
                 const int wq = issue_M(C, k, issue_V(C, k, 0));
                 const int ql = uni(S.cs_ptr[k + 1]) - 1;
-                if (ql == uni(S.cs_ptr[k]) && uni(S.first[S.cs_idx[ql]]) == k - 1) {
+                if (ql >= uni(S.cs_ptr[k]) && uni(S.first[S.cs_idx[ql]]) == k - 1) {
                     const int tn = C.tv[k], wn = C.wv[k];
                     issue_G(C, k - 1, C.Lk(k - 1), C.ts + C.sl.G, 2 * tn, tn, (long)wn * 2 * tn, wq);
                     nn_ready = true;
@@ -737,9 +737,11 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
             }
             if constexpr (!CH) advance_M(C, k);
         }
-        const int q0 = uni(S.cs_ptr[k]), nq = uni(S.cs_ptr[k + 1]) - q0;
-        if (nq == 1 && uni(S.first[S.cs_idx[q0]]) == k - 1) {
-            const int c = S.cs_idx[q0], i = k - 1;
+        const int q0 = uni(S.cs_ptr[k]), nall = uni(S.cs_ptr[k + 1]) - q0;
+        const bool nn = nall > 0 && uni(S.first[S.cs_idx[q0 + nall - 1]]) == k - 1;
+        const int nq = nn ? nall - 1 : nall;
+        if (nn) {
+            const int c = uni(S.cs_idx[q0 + nq]), i = k - 1;
             const int tn = C.tv[i + 1], wn = C.wv[i + 1];
             const T *g[4];
             if (!nn_ready) compute_G(C, i, C.Lk(i));
@@ -749,14 +751,18 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
                 g[ch] = G + (size_t)sp * tn + (size_t)s * wn * 2 * tn;
             }
             pair_tensor(C, C.tv[k], C.wv[k], g, 2 * tn, M, r_pending ? C.Rk(k) : nullptr);
+            r_pending = false;
             double e = 0.0;
             for (int q2 = 0; q2 < 16; ++q2) e += S.SS[q2] * M[q2];
             etot += S.Jc[c] * e;
-        } else if (nq > 0) {
-            // only sum_i J_ik S_i . S_k is needed: the operator channels S^z, S^+, S^-
+        }
+        if (nq > 0) {
+            // long range: only sum_i J_ik S_i . S_k is needed: the operator channels S^z, S^+, S^-
             // of site i (ch = 2 s' + s: S^z = (G(1,1) - G(0,0)) / 2, S^+ = G(1,0),
             // S^- = G(0,1)) times J_ik start at the leftmost partner of k, take in
-            // each further one on their way right, and meet V once at bond k
+            // each further one on their way right, and meet V once at bond k (the FP32
+            // sum costs nothing: relative error of the energy of 64 walkers near the 4x4
+            // torus' trial at D = 20 against FP64 2.0e-7 either way)
             T *A = C.ts + C.sl.GcA, *B = C.ts + C.sl.GcB;
             int bond = -1;
             for (int q = q0; q <= q0 + nq; ++q) {
