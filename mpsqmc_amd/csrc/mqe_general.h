@@ -8,16 +8,6 @@
 
 namespace mqe {
 
-// Wave-uniform values.  Bond dimensions, site numbers and the tensors' addresses
-// are the same in every lane of a workgroup, but the compiler cannot know it of
-// values that come from LDS or memory: held in vector registers they made every
-// loop bound a lane mask, every address 64-bit vector arithmetic and every buffer
-// resource a loop over the lanes' values.
-__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
-__device__ __forceinline__ long uni(long x) {
-    const unsigned lo = (unsigned)uni((int)(unsigned)x), hi = (unsigned)uni((int)(unsigned)((unsigned long)x >> 32));
-    return (long)(((unsigned long)hi << 32) | lo);
-}
 struct UniDims {  // bond dimensions in LDS, read as uniform values
     const int *p;
     __device__ __forceinline__ int operator[](int k) const { return uni(p[k]); }
@@ -39,8 +29,7 @@ struct Ctx {
     T *ts;               // T scratch
     double *ds;          // double scratch
     double *red;         // LDS reduction scratch (>= MQE_NT + 16*MQE_WAVES)
-    double *qlds;        // LDS workspace of the LQ (tau, then trailing columns), or nullptr
-    long qlds_doubles;   // its size
+    long qlds_doubles;   // dynamic LDS: the workspace of the LQ (0: none)
     int tile;            // output tile shape of the FP32 matrix-core products (TILE_*)
 
     const float *trialT; // FP32: the trial with every T_k[s] transposed (t_{k+1} x t_k), or nullptr
@@ -572,36 +561,44 @@ __device__ __forceinline__ void apply_op(const Ctx<T, CH> &C, int k, const doubl
     __syncthreads();
 }
 
-// LQ of site k (w_k x 2 w_{k+1}) in FP64: phi_k <- Q (right-orthonormal),
-// phi_{k-1} <- phi_{k-1} Lmat, then R_k = sum_t T_k[t] R_{k+1} Q[t]^T.
-// Leaves V (all four blocks) computed for bond k.
+// FP64 LQ of a site ph (wk x 2 wn): ph <- Q (right-orthonormal), LM <- Lmat (wk x wk).
 // The factorisation is a serial chain of column steps; it runs with every
-// column in registers where the site fits (at most 128 x 64, reflectors in LDS)
-// and over columns in LDS and memory above.  One step of 200 walkers of a 15-site
+// column in registers where the site fits (at most 128 x 64, reflectors in LDS),
+// by panels of 32 columns in registers up to 256 x 128, and over columns in LDS
+// and memory above.  One step of 200 walkers of a 15-site
 // ring in a field at D = 20 (two sweeps of LQ): 2121 us with the columns in LDS,
 // 1634 us in registers; 128 walkers of 16 sites at D = 16 in FP64, where one or
 // two walkers a step take this sweep and the others wait: 1230 and 1042 us.
+// A function of its own, not inlined: its register columns in the kernel's body
+// made the products of the other walkers spill (a step of the 6x6 snake at D = 128
+// without canonical walkers 115 ms, 134 ms with the panels inlined).
+// AQ, RQ, TAU: the walker's scratch; nq: doubles of dynamic LDS.
 template <typename T, bool CH>
-__device__ __forceinline__ void lq_site(const Ctx<T, CH> &C, int k) {
-    const int wk = C.wv[k], wn = C.wv[k + 1], wp = C.wv[k - 1];
+__device__ __noinline__ void lq_factor(T *ph_, T *LM_, double *AQ_, double *RQ_, double *TAU_, int wk_, int wn_,
+                                       int Dw, int nq) {
+    extern __shared__ double qlds_dyn[];
+    constexpr bool PANELS = !CH;  // (chained: every bond is at most 64)
+    const int wk = uni(wk_), wn = uni(wn_);
+    T *ph = (T *)uni((long)ph_), *LM = (T *)uni((long)LM_);
+    double *AQ = (double *)uni((long)AQ_);
+    nq = uni(nq);
     const int m = 2 * wn, n = wk;
-    T *ph = C.site(k);
-    T *LM = C.ts + C.sl.LM;
-    if (C.qlds && n <= m && m <= QR_REGS_M && n <= QR_REGS_N &&
-        C.qlds_doubles >= (m <= 64 && n <= 32 ? 65L : 129L) * n) {
-        qr_in_regs(
-            m, n, C.qlds + n, C.qlds, true, [&](int r, int c) { return (double)ph[c + (size_t)wk * r]; },
-            [&](int r, int c, double x) {
-                LM[c + (size_t)n * r] = (T)x;
-                if (r != c) LM[r + (size_t)n * c] = T(0);
-            },
-            [&](int r, int c, double x) { ph[c + (size_t)wk * r] = (T)x; });
+    auto load = [&](int r, int c) { return (double)ph[c + (size_t)wk * r]; };
+    auto put_r = [&](int r, int c, double x) {  // Lmat = R^T
+        LM[c + (size_t)n * r] = (T)x;
+        if (r != c) LM[r + (size_t)n * c] = T(0);
+    };
+    auto put_q = [&](int r, int c, double x) { ph[c + (size_t)wk * r] = (T)x; };
+    const bool fits = nq > 0 && n <= m;
+    if (fits && m <= QR_REGS_M && n <= QR_REGS_N && nq >= (m <= 64 && n <= 32 ? 65 : 129) * n) {
+        qr_in_regs(m, n, qlds_dyn + n, qlds_dyn, true, load, put_r, put_q);
+    } else if (PANELS && fits && m <= QR_PANELS_M && n <= QR_PANELS_N && nq >= QR_PANELS_M * QR_PANEL + n) {
+        qr_panels(m, n, qlds_dyn + n, qlds_dyn, AQ, load, put_r, put_q);
     } else {
-        double *R = C.ds + C.sl.RQ;
-        double *tau = C.qlds ? C.qlds : C.ds + C.sl.TAU;
-        int nl = 0;
-        if (C.qlds) nl = min(n, (int)((C.qlds_doubles - C.S->Dw) / m));
-        const QRCols col{C.ds + C.sl.AQ, C.qlds ? C.qlds + C.S->Dw : nullptr, m, n - nl};
+        double *R = (double *)uni((long)RQ_);
+        double *tau = nq > 0 ? qlds_dyn : (double *)uni((long)TAU_);
+        const int D = uni(Dw), nl = nq > 0 ? min(n, (nq - D) / m) : 0;
+        const QRCols col{AQ, nq > 0 ? qlds_dyn + D : nullptr, m, n - nl};
         for (int e = threadIdx.x; e < m * n; e += MQE_NT) {
             const int r = e % m, c = e / m;
             col(c)[r] = (double)ph[c + (size_t)wk * r];
@@ -618,6 +615,16 @@ __device__ __forceinline__ void lq_site(const Ctx<T, CH> &C, int k) {
         }
     }
     __syncthreads();
+}
+
+// LQ of site k: phi_k <- Q, phi_{k-1} <- phi_{k-1} Lmat, then
+// R_k = sum_t T_k[t] R_{k+1} Q[t]^T.  Leaves V (all four blocks) computed for bond k.
+template <typename T, bool CH>
+__device__ __forceinline__ void lq_site(const Ctx<T, CH> &C, int k) {
+    const int wk = C.wv[k], wn = C.wv[k + 1], wp = C.wv[k - 1];
+    T *LM = C.ts + C.sl.LM;
+    lq_factor<T, CH>(C.site(k), LM, C.ds + C.sl.AQ, C.ds + C.sl.RQ, C.ds + C.sl.TAU, wk, wn, C.S->Dw,
+                     (int)C.qlds_doubles);
     // push Lmat into the left neighbour
     T *pl = C.site(k - 1), *tmp = C.ts + C.sl.TMP;
     gemm_batch<false, false, T>(2, wp, wk, wk, pl, wp, (long)wp * wk, LM, wk, 0, tmp, wp, (long)wp * wk, false, C.tile);
@@ -968,8 +975,6 @@ __global__ __launch_bounds__(MQE_NT, 2) void walker_kernel(Sys S, Pool P, const 
     long tb = (C.sl.t_total * (long)sizeof(T) + 255) & ~255L;
     C.ds = (double *)(base + tb);
     C.red = red;
-    extern __shared__ double qlds_dyn[];
-    C.qlds = P.qlds > 0 ? qlds_dyn : nullptr;
     C.qlds_doubles = P.qlds;
 
     double w = P.w[slot];

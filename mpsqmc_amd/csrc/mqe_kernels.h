@@ -112,7 +112,8 @@ __host__ __device__ inline ScratchLayout scratch_layout(int Dt, int Dw, int Ng) 
     s.LM = o; o += (long)Dw * Dw;
     s.t_total = o;
     o = 0;
-    s.AQ = o; o += 2L * Dw * Dw;
+    const long panels = Dw <= QR_PANELS_N ? panel_doubles((int)Dw) : 0;  // the LQ's reflectors
+    s.AQ = o; o += 2L * Dw * Dw > panels ? 2L * Dw * Dw : panels;
     s.RQ = o; o += (long)Dw * Dw;
     s.TAU = o; o += Dw;
     s.PARTS = o; o += MQE_NT;

@@ -1,5 +1,6 @@
-"""The canonical sweep's LQ at the edges of its two forms: in registers up to a
-128 x 64 site (8 lanes a column up to 64 x 32, else 4), in memory above.  Energy,
+"""The canonical sweep's LQ at the edges of its three forms: in registers up to a
+128 x 64 site (8 lanes a column up to 64 x 32, else 4), by panels of 32 columns up
+to 256 x 128, in memory above.  Energy,
 overlap and the right-orthonormality of every site against the oracle and plain
 numpy; bars 1e-10 as for the other FP64 quantities (LQ errors are a few ulps a
 site, the bar leaves four orders of magnitude)."""
@@ -15,9 +16,10 @@ from .common import oracle_population, random_trial, rel
 pytestmark = [pytest.mark.gpu, pytest.mark.usefixtures("require_gpu")]
 
 
-@pytest.mark.parametrize("L,D", [(3, 2), (6, 3), (11, 31), (12, 32), (12, 33), (13, 63), (13, 64), (14, 65)])
+@pytest.mark.parametrize("L,D", [(3, 2), (6, 3), (11, 31), (12, 32), (12, 33), (13, 63), (13, 64), (14, 65),
+                                 (15, 97), (16, 128), (17, 130)])
 def test_prepare_shapes_fp64(L, D):
-    s = systems.chain(L, periodic=L > 4)
+    s = systems.chain(L, periodic=4 < L < 14)
     tvd, tdata = random_trial(L, D, L + D)
     n = 3
     orc = oracle_population(s, tvd, tdata)
