@@ -272,6 +272,35 @@ __device__ __forceinline__ void mfma_step(float a, float b, float (&c)[TileGeom<
     for (int e = 0; e < TileGeom<TS>::NACC; ++e) c[e] = x[e];
 }
 
+// Buffer resources over one walker's or the trial's arrays: the 64-bit base in
+// scalar registers and 32-bit byte offsets per lane.  An offset at or beyond
+// BUF_RANGE reads 0 and drops a store (the hardware range check).
+constexpr int BUF_RANGE = 0x7ffffff0;
+constexpr int BUF_OOB = 0x7ffffff8;
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p) {
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, BUF_RANGE, 0x00020000);
+}
+// (the b32 / b128 builtins move raw 32-bit words: bit casts, not conversions)
+template <typename T = float>
+__device__ __forceinline__ T buf_ld(__amdgpu_buffer_rsrc_t r, int voff) {
+    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
+    else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
+}
+__device__ __forceinline__ void buf_st(float v, __amdgpu_buffer_rsrc_t r, int voff, int imm) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, voff, imm, 0);
+}
+__device__ __forceinline__ void buf_st(double v, __amdgpu_buffer_rsrc_t r, int voff, int imm) {
+    typedef unsigned int u2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, voff, imm, 0);
+}
+__device__ __forceinline__ void buf_ld4(__amdgpu_buffer_rsrc_t r, int voff, float *v) {
+    const float4 x = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
+    v[0] = x.x;
+    v[1] = x.y;
+    v[2] = x.z;
+    v[3] = x.w;
+}
+
 // k a positive multiple of 16: every wave runs one pipelined chain over the
 // (tile, term, slice) items of its tiles.  The operands of the item two ahead
 // are loaded unconditionally (past the end the last item reloads itself) with
@@ -336,6 +365,140 @@ __device__ __forceinline__ void gemm_tiles_full(int m, int n, int k, const float
     }
 }
 
+// Run of NV operand values of a slice through a buffer resource: voff the lane's
+// byte offset, soff the slice's, step the bytes per k (stored across k), left the
+// values of the lane's run inside the matrix (TAIL: the others read 0).
+template <bool KC, bool VEC, bool TAIL, int NV>
+__device__ __forceinline__ void load_run_buf(__amdgpu_buffer_rsrc_t r, int voff, int soff, int step, int left,
+                                             float (&v)[NV]) {
+    if constexpr (KC && VEC) {
+#pragma unroll
+        for (int j = 0; j < NV / 4; ++j) {
+            const float4 x = __builtin_bit_cast(
+                float4, __builtin_amdgcn_raw_buffer_load_b128(r, !TAIL || 4 * j < left ? voff + 16 * j : BUF_OOB, soff, 0));
+            v[4 * j] = x.x;
+            v[4 * j + 1] = x.y;
+            v[4 * j + 2] = x.z;
+            v[4 * j + 3] = x.w;
+        }
+    } else {
+#pragma unroll
+        for (int u = 0; u < NV; ++u) {
+            const int o = KC ? voff + 4 * u : voff;
+            v[u] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(r, !TAIL || u < left ? o : BUF_OOB,
+                                                                                 KC ? soff : soff + step * u, 0));
+        }
+    }
+}
+
+// The same chain for operands in global memory with uniform shapes (bonds above
+// 64): a cursor in scalar registers steps through the (tile, term, slice) items,
+// each load is one instruction (scalar slice offset, the lane's offset of the
+// tile), and a last partial slice reads zeros past k.  One wave per SIMD has to
+// issue everything between its MFMAs itself: with the operand addresses formed
+// from the item's number per load (divisions, 64-bit vector arithmetic) a step of
+// 256 walkers of the 6x6 snake at D = 128 took 151 ms, with the cursor 141 ms in
+// 32 x 32 and 130 ms in 32 x 64 tiles.
+// VEC: operands stored along k are 16-byte aligned and k is a multiple of 4.
+template <bool TA, bool TB, int TS, int NW, bool VEC>
+__device__ __forceinline__ void gemm_tiles_buf(int m, int n, int k, const float *A0, const float *A1, int lda,
+                                             const float *B0, const float *B1, int ldb, float *C0, int ldc, bool acc,
+                                             int nseg, int nb, long sA, long sB, long sC) {
+    constexpr int KL = TileGeom<TS>::KL, NACC = TileGeom<TS>::NACC;
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane % TS, h = lane / TS;
+    const int tm = (m + TS - 1) / TS, tn = (n + TS * NW - 1) / (TS * NW), ntile = nb * tm * tn;
+    if (w >= ntile) return;
+    const int ntw = (ntile - w + MQE_WAVES - 1) / MQE_WAVES;  // tiles of this wave
+    const int nsk = (k + 15) >> 4, nsl = nseg * nsk, nit = ntw * nsl;
+    const int stA = TA ? 4 : 4 * lda, stB = TB ? 4 * ldb : 4;  // bytes per k
+    // cursor: tile j, term seg, slice sl
+    int j = 0, seg = 0, sl = 0, va = 0, vb[NW], bt = 0;
+    __amdgpu_buffer_rsrc_t ra, rb;
+    auto base = [&]() {
+        ra = buf_rsrc((seg ? A1 : A0) + (size_t)bt * sA);
+        rb = buf_rsrc((seg ? B1 : B0) + (size_t)bt * sB);
+    };
+    auto tile = [&]() {
+        const int tb = w + MQE_WAVES * j;
+        bt = tb / (tm * tn);
+        const int t = tb - bt * (tm * tn), tq = t / tm;
+        const int ar = min((t - tq * tm) * TS + r, m - 1);
+        va = TA ? 4 * (lda * ar + KL * h) : 4 * (ar + lda * KL * h);
+#pragma unroll
+        for (int q = 0; q < NW; ++q) {
+            const int bc = min(tq * TS * NW + TS * q + r, n - 1);
+            vb[q] = TB ? 4 * (bc + ldb * KL * h) : 4 * (ldb * bc + KL * h);
+        }
+        base();
+    };
+    tile();
+    auto load = [&](float (&a)[KL], float (&b)[NW][KL]) {
+        const int oa = stA * 16 * sl, ob = stB * 16 * sl;
+        if (16 * sl + 16 <= k) {
+            load_run_buf<TA, VEC, false, KL>(ra, va, oa, stA, 0, a);
+#pragma unroll
+            for (int q = 0; q < NW; ++q) load_run_buf<!TB, VEC, false, KL>(rb, vb[q], ob, stB, 0, b[q]);
+        } else {
+            const int left = k - 16 * sl - KL * h;
+            load_run_buf<TA, VEC, true, KL>(ra, va, oa, stA, left, a);
+#pragma unroll
+            for (int q = 0; q < NW; ++q) load_run_buf<!TB, VEC, true, KL>(rb, vb[q], ob, stB, left, b[q]);
+        }
+        // next item (the last one repeats: its loads are not used)
+        if (++sl == nsk) {
+            if (seg + 1 < nseg) {
+                ++seg;
+                sl = 0;
+                base();
+            } else if (j + 1 < ntw) {
+                ++j;
+                seg = sl = 0;
+                tile();
+            } else {
+                sl = nsk - 1;
+            }
+        }
+    };
+    float a0[KL], b0[NW][KL], a1[KL], b1[NW][KL], a2[KL], b2[NW][KL], c[NW][NACC];
+#pragma unroll
+    for (int q = 0; q < NW; ++q)
+#pragma unroll
+        for (int e = 0; e < NACC; ++e) c[q][e] = 0.f;
+    int done = 0, tdone = w;  // slices of the tile being summed, its number
+    auto step = [&](const float (&a)[KL], const float (&b)[NW][KL]) {
+#pragma unroll
+        for (int u = 0; u < KL; ++u)
+#pragma unroll
+            for (int q = 0; q < NW; ++q) mfma_step<TS>(a[u], b[q][u], c[q]);
+        if (++done == nsl) {  // the tile is complete
+            tile_store<TS, NW>(C0, ldc, sC, tdone, m, n, tm, tn, r, h, acc, c);
+            done = 0;
+            tdone += MQE_WAVES;
+#pragma unroll
+            for (int q = 0; q < NW; ++q)
+#pragma unroll
+                for (int e = 0; e < NACC; ++e) c[q][e] = 0.f;
+        }
+    };
+    load(a0, b0);
+    load(a1, b1);
+#pragma nounroll
+    for (int i = 0; i < nit; i += 3) {
+        load(a2, b2);
+        __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of the MFMAs
+        step(a0, b0);
+        if (i + 1 >= nit) break;
+        load(a0, b0);
+        __builtin_amdgcn_sched_barrier(0);
+        step(a1, b1);
+        if (i + 2 >= nit) break;
+        load(a1, b1);
+        __builtin_amdgcn_sched_barrier(0);
+        step(a2, b2);
+    }
+}
+
 // Any k: per tile and slice, predicated loads (zeros at k >= k), no pipelining.
 template <bool TA, bool TB, int TS, int NW>
 __device__ __forceinline__ void gemm_tiles_pred(int m, int n, int k, const float *A0, const float *A1, int lda,
@@ -397,17 +560,29 @@ __device__ __forceinline__ void gemm_mfma(int m, int n, int k, const float *A0, 
 // bucket by the engine's tile table).
 enum : int { TILE_16 = 16, TILE_32 = 32, TILE_WIDE = 64 };
 
-// The matrix-core product with the output tile shape `tile`.
+// The matrix-core product with the output tile shape `tile` (uniform shapes and
+// addresses, operands in global memory).
+template <bool TA, bool TB, int TS, int NW>
+__device__ __forceinline__ void gemm_shape(int m, int n, int k, const float *A0, const float *A1, int lda,
+                                           const float *B0, const float *B1, int ldb, float *C, int ldc, bool acc,
+                                           int nseg, int nb, long sA, long sB, long sC) {
+    const bool vec = (k & 3) == 0 && (!TA || aligned16(A0, nseg > 1 ? A1 : A0, lda, sA)) &&
+                     (TB || aligned16(B0, nseg > 1 ? B1 : B0, ldb, sB));
+    if (vec)
+        gemm_tiles_buf<TA, TB, TS, NW, true>(m, n, k, A0, A1, lda, B0, B1, ldb, C, ldc, acc, nseg, nb, sA, sB, sC);
+    else
+        gemm_tiles_buf<TA, TB, TS, NW, false>(m, n, k, A0, A1, lda, B0, B1, ldb, C, ldc, acc, nseg, nb, sA, sB, sC);
+}
 template <bool TA, bool TB>
 __device__ __forceinline__ void gemm_f32(int m, int n, int k, const float *A0, const float *A1, int lda,
                                          const float *B0, const float *B1, int ldb, float *C, int ldc, bool acc,
                                          int nseg, int nb, long sA, long sB, long sC, int tile) {
     if (tile == TILE_16)
-        gemm_tiles<TA, TB, 16, 1>(m, n, k, A0, A1, lda, B0, B1, ldb, C, ldc, acc, nseg, nb, sA, sB, sC);
+        gemm_shape<TA, TB, 16, 1>(m, n, k, A0, A1, lda, B0, B1, ldb, C, ldc, acc, nseg, nb, sA, sB, sC);
     else if (tile == TILE_WIDE && n > 32)
-        gemm_tiles<TA, TB, 32, 2>(m, n, k, A0, A1, lda, B0, B1, ldb, C, ldc, acc, nseg, nb, sA, sB, sC);
+        gemm_shape<TA, TB, 32, 2>(m, n, k, A0, A1, lda, B0, B1, ldb, C, ldc, acc, nseg, nb, sA, sB, sC);
     else
-        gemm_tiles<TA, TB, 32, 1>(m, n, k, A0, A1, lda, B0, B1, ldb, C, ldc, acc, nseg, nb, sA, sB, sC);
+        gemm_shape<TA, TB, 32, 1>(m, n, k, A0, A1, lda, B0, B1, ldb, C, ldc, acc, nseg, nb, sA, sB, sC);
 }
 
 // Vector-unit product (FP64, and FP32 products too small for the matrix cores).
@@ -520,35 +695,6 @@ typedef float v16f_c __attribute__((ext_vector_type(16)));
 
 __device__ __forceinline__ v16f_c mfma32(float a, float b, v16f_c c) {
     return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0);
-}
-
-// Buffer resources over one walker's or the trial's arrays: the 64-bit base in
-// scalar registers and 32-bit byte offsets per lane.  An offset at or beyond
-// BUF_RANGE reads 0 and drops a store (the hardware range check).
-constexpr int BUF_RANGE = 0x7ffffff0;
-constexpr int BUF_OOB = 0x7ffffff8;
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t buf_rsrc(const void *p) {
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), 0, BUF_RANGE, 0x00020000);
-}
-// (the b32 / b128 builtins move raw 32-bit words: bit casts, not conversions)
-template <typename T = float>
-__device__ __forceinline__ T buf_ld(__amdgpu_buffer_rsrc_t r, int voff) {
-    if constexpr (sizeof(T) == 8) return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, voff, 0, 0));
-    else return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b32(r, voff, 0, 0));
-}
-__device__ __forceinline__ void buf_st(float v, __amdgpu_buffer_rsrc_t r, int voff, int imm) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned int, v), r, voff, imm, 0);
-}
-__device__ __forceinline__ void buf_st(double v, __amdgpu_buffer_rsrc_t r, int voff, int imm) {
-    typedef unsigned int u2 __attribute__((ext_vector_type(2)));
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u2, v), r, voff, imm, 0);
-}
-__device__ __forceinline__ void buf_ld4(__amdgpu_buffer_rsrc_t r, int voff, float *v) {
-    const float4 x = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(r, voff, 0, 0));
-    v[0] = x.x;
-    v[1] = x.y;
-    v[2] = x.z;
-    v[3] = x.w;
 }
 
 // qsplit: the two row tiles of D are separate items (the F strips formed for
