@@ -839,6 +839,8 @@ __device__ __forceinline__ int chain2(int wave0, int nu, int m1, int n1, int k1,
 // (a bond of 48 in three 16-column strips re-reads A and C three times and
 // measured 20 % slower than two 32-column strips).
 // qsplit: the D row tiles 0-1 and 2-3 are separate items.
+// SEP (NF = 2): the two terms of D are summed by themselves and then added
+// (shorter sums, a smaller rounding error, sixteen more registers).
 // FP64 (v_mfma_f64_16x16x4f64) takes all bonds up to 64 this way.  Its
 // accumulator slot e of lane (c, g) holds row g + 4e, so MFMA e of F tile t in
 // the second chain takes rows 16t + g + 4e.  The general products' vector-unit
@@ -867,7 +869,7 @@ struct Chain16<double> {
     static constexpr int ROW_G = 1, ROW_E = 4;
 };
 
-template <bool TB, bool TC, int NF, int ND, typename T, class Get>
+template <bool TB, bool TC, int NF, int ND, typename T, bool SEP = false, class Get>
 __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int k1, int mD, int lda, int ldb, int ldc,
                                          int ldd, bool qsplit, Get get) {
     typedef Chain16<T> CT;
@@ -887,7 +889,7 @@ __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int 
         const int q0 = nq == 1 ? 0 : 2 * qi, q1 = nq == 1 ? QT : min(QT, 2 * qi + 2);  // D row tiles of this item
         const ChainOps<T> op = get(u);
         int c = lane & 15, g = lane >> 4;
-        V4 D[4];
+        V4 D[4], D0[SEP ? 4 : 1];
 #pragma nounroll
         for (int f = 0; f < NF; ++f) {
             asm volatile("" : "+v"(c), "+v"(g));
@@ -935,7 +937,11 @@ __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int 
                 const T *Cp = (ND == 1 ? f : d) == 0 ? op.C[0] : op.C[1];
                 const auto rC = buf_rsrc(Cp);
                 const bool vecC = TC && SZ == 4 && (m1 & 3) == 0 && (ldc & 3) == 0 && (((uintptr_t)Cp) & 15u) == 0;
-                if (ND == 2 || f == 0) {
+                if (SEP && f == 1) {
+#pragma unroll
+                    for (int qd = 0; qd < 4; ++qd) D0[SEP ? qd : 0] = D[qd];
+                }
+                if (SEP || ND == 2 || f == 0) {
 #pragma unroll
                     for (int qd = 0; qd < 4; ++qd) D[qd] = V4{0, 0, 0, 0};
                 }
@@ -967,6 +973,10 @@ __device__ __forceinline__ int chain2_16(int wave0, int nu, int m1, int n1, int 
                             D[qd] = CT::mfma(cv[t][e], F[t][e], D[qd]);
                         }
                     }
+                }
+                if (SEP && f == 1) {
+#pragma unroll
+                    for (int qd = 0; qd < 4; ++qd) D[qd] += D0[SEP ? qd : 0];
                 }
                 if (f == NF - 1) {
                     // row 16 qd + row(g, e) of column c0 + c; outside D the store is dropped

@@ -51,7 +51,11 @@ static thread_local std::string g_err;
 void set_error(const char *msg) { g_err = msg ? msg : ""; }
 
 // out[b] = <other | walker_b> (transfer matrices, MPSstate.cpp:248-284).
-template <typename T>
+// CH (every bond of both states at most 64): the two products of a site are
+// chained in registers (one barrier per site); what bounds it is the latency of
+// a site's loads and its dependent products.  1024 walkers of 32 sites, bonds 32
+// and 24: 384 us with three products and barriers per site, @O@ us chained.
+template <typename T, bool CH>
 __global__ __launch_bounds__(MQE_NT) void overlap_kernel(int L, const int *ovd, const long *ooff, const T *other,
                                                        Pool P, int Dmax, double *out, int first) {
     const int b = first + blockIdx.x;  // population position; workspace blockIdx.x of P.scratch
@@ -74,6 +78,27 @@ __global__ __launch_bounds__(MQE_NT) void overlap_kernel(int L, const int *ovd, 
         const T *B0 = P.padded ? phi + (size_t)(2 * k) * 1024 : phi + uni(P.woff[k]);
         const T *B1 = P.padded ? phi + (size_t)(2 * k + 1) * 1024 : B0 + (size_t)wa * wb;
         const int ldb = P.padded ? 32 : wa;
+        if constexpr (CH) {
+            auto unit = [&](int) {
+                ChainOps<T> o;
+                o.A = E;
+                o.B[0] = A;
+                o.B[1] = A + (size_t)oa * ob;
+                o.C[0] = B0;
+                o.C[1] = B1;
+                o.D[0] = o.D[1] = E2;
+                return o;
+            };
+            bool wide = false;
+            if constexpr (sizeof(T) == sizeof(float)) {
+                wide = ob > 32;  // two 32-column strips, else 16-column ones
+                if (wide) chain2<false, true, 2, 1>(0, 1, wa, ob, oa, wb, wa, oa, ldb, wb, true, unit);
+            }
+            if (!wide) chain2_16<false, true, 2, 1, T, true>(0, 1, wa, ob, oa, wb, wa, oa, ldb, wb, true, unit);
+            __syncthreads();
+            T *t = E; E = E2; E2 = t;
+            continue;
+        }
         // Y = E A (wa x 2 ob) with E (wa x oa)
         gemm<false, false, T>(wa, 2 * ob, oa, E, wa, A, oa, Y, wa, false);
         __syncthreads();
@@ -1041,6 +1066,20 @@ int overlaps_workspace(mqe_engine *e, const mqe_mps *other, long *bytes_all, lon
     return MQE_OK;
 }
 
+// `other` in the engine's precision; Dmax: the largest bond of the walkers and it
+static void launch_overlap(mqe_engine *e, dim3 grid, const int *ovd, const long *ooff, const void *other, const Pool &P,
+                           int Dmax, int first) {
+    auto go = [&](auto kernel, auto *o) {
+        hipLaunchKernelGGL(kernel, grid, dim3(MQE_NT), 0, e->stream, e->L, ovd, ooff, o, P, Dmax, e->d_tmpout, first);
+    };
+    const float *of = (const float *)other;
+    const double *od = (const double *)other;
+    if (e->fp32 && Dmax <= 64) go(overlap_kernel<float, true>, of);
+    else if (e->fp32) go(overlap_kernel<float, false>, of);
+    else if (Dmax <= 64) go(overlap_kernel<double, true>, od);
+    else go(overlap_kernel<double, false>, od);
+}
+
 int overlaps_in_workspace(mqe_engine *e, const mqe_mps *other, double *out, char *ws, long ws_bytes) {
     OverlapPlan pl;
     ECHK(plan_overlaps(e, other, &pl));
@@ -1061,9 +1100,10 @@ int overlaps_in_workspace(mqe_engine *e, const mqe_mps *other, double *out, char
         t += (long)other->vd[k] * other->vd[k + 1] * 2;
     }
     if (e->fp32) {
-        float tmp[4096];
-        for (long i0 = 0; i0 < pl.tot; i0 += 4096) {
-            const long m = std::min(4096L, pl.tot - i0);
+        constexpr long CHUNK = 32768;  // a synchronous copy costs about 10 us whatever its size here
+        float tmp[CHUNK];
+        for (long i0 = 0; i0 < pl.tot; i0 += CHUNK) {
+            const long m = std::min(CHUNK, pl.tot - i0);
             for (long i = 0; i < m; ++i) tmp[i] = (float)other->data[i0 + i];
             HIPCHK(hipMemcpy(ws + sizeof(float) * i0, tmp, sizeof(float) * m, hipMemcpyHostToDevice));
         }
@@ -1078,12 +1118,7 @@ int overlaps_in_workspace(mqe_engine *e, const mqe_mps *other, double *out, char
     const int *ovd = (const int *)(ws + pl.off_vd);
     const long *ooff = (const long *)(ws + pl.off_off);
     for (int f = 0; f < n; f += chunk) {
-        if (e->fp32)
-            hipLaunchKernelGGL(overlap_kernel<float>, dim3(chunk), dim3(MQE_NT), 0, e->stream, L, ovd, ooff,
-                               (const float *)ws, P, pl.Dmax, e->d_tmpout, f);
-        else
-            hipLaunchKernelGGL(overlap_kernel<double>, dim3(chunk), dim3(MQE_NT), 0, e->stream, L, ovd, ooff,
-                               (const double *)ws, P, pl.Dmax, e->d_tmpout, f);
+        launch_overlap(e, dim3(chunk), ovd, ooff, ws, P, pl.Dmax, f);
         HIPCHK(hipGetLastError());
     }
     HIPCHK(hipStreamSynchronize(e->stream));
@@ -1999,13 +2034,11 @@ int mqe_compress_walkers(mqe_engine *e, const int *targets) {
     HIPCHK(hipMalloc((void **)&scr, need * std::max(n, 1)));
     P.scratch = scr;
     P.scratch_bytes = (long)need;
+    launch_overlap(e, dim3(n), e->d_tvd, e->d_toff, e->d_trial, P, Do, 0);
+    HIPCHK(hipGetLastError());
     if (e->fp32) {
-        hipLaunchKernelGGL(overlap_kernel<float>, dim3(n), dim3(MQE_NT), 0, e->stream, L, e->d_tvd, e->d_toff,
-                           (const float *)e->d_trial, P, Do, e->d_tmpout, 0);
         hipLaunchKernelGGL(overlap_sign_kernel<float>, dim3(n), dim3(64), 0, e->stream, L, P, e->d_tmpout, dt);
     } else {
-        hipLaunchKernelGGL(overlap_kernel<double>, dim3(n), dim3(MQE_NT), 0, e->stream, L, e->d_tvd, e->d_toff,
-                           (const double *)e->d_trial, P, Do, e->d_tmpout, 0);
         hipLaunchKernelGGL(overlap_sign_kernel<double>, dim3(n), dim3(64), 0, e->stream, L, P, e->d_tmpout, dt);
     }
     HIPCHK(hipGetLastError());
