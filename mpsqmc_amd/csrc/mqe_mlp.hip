@@ -7,7 +7,7 @@
 // the prediction into a proposal over the grid and corrects the weight with the
 // exact PDF value of the sampled point.  The reference has no such component.
 //
-// Kernels: one workgroup per tile of 64 samples.  The activations of a tile
+// Kernels: one workgroup per tile of 32 samples.  The activations of a tile
 // stay in LDS (feature-major, ld = width); every layer product is a workgroup
 // MFMA GEMM (v_mfma_f32_32x32x2f32) with the weights read from global memory
 // (80 KB at H = 128, L2-resident).  Training computes forward and backward of a
@@ -33,7 +33,11 @@
 namespace mqe {
 namespace mlp {
 
-constexpr int TS = 64;         // samples per tile
+// Samples per tile.  What bounds a tile is the latency of its layers, one after the
+// other; with 32 samples (instead of 64) four tiles share a CU and every wave has one
+// output tile per layer: forward of 63,488 rows at H = 128 107 -> 93 us, gradient of
+// 16,384 rows 88 -> 79 us; with the padded blocks below 80 and 71 us.
+constexpr int TS = 32;
 constexpr int MAX_IN = 32, MAX_H = 128, MAX_OUT = 32;
 
 struct Net {
@@ -49,16 +53,24 @@ __host__ __device__ inline long off_W3(int nin, int H) { return off_b2(nin, H) +
 __host__ __device__ inline long off_b3(int nin, int H, int nout) { return off_W3(nin, H) + (long)nout * H; }
 __host__ __device__ inline long num_params(int nin, int H, int nout) { return off_b3(nin, H, nout) + nout; }
 
+// Leading dimension of an activation block of `rows` features in LDS.  The layer
+// products read it along the features, one sample per lane: with the feature count
+// itself (128) every lane of a read fell on the same banks.  A multiple of four
+// (16-byte reads) that is four past one of the block's size spreads 16 samples
+// over all 64 banks.
+__host__ __device__ inline int act_ld(int rows) { return ((rows + 3) & ~3) + 4; }
+
 inline size_t lds_bytes(int nin, int H, int nout, bool train) {
     // xs [nin x TS], h1, h2 [H x TS], o [nout x TS], (train) dh2 [H x TS]
-    return sizeof(float) * (size_t)TS * (nin + 2 * H + nout + (train ? H : 0));
+    return sizeof(float) * (size_t)TS * (nin + 2 * act_ld(H) + act_ld(nout) + (train ? act_ld(H) : 0));
 }
 
 // bias + optional ReLU on a [rows x TS] LDS block
-__device__ __forceinline__ void bias_act(float *a, int rows, const float *b, bool relu) {
+__device__ __forceinline__ void bias_act(float *a, int rows, int ld, const float *b, bool relu) {
     for (int e = threadIdx.x; e < rows * TS; e += MQE_NT) {
-        float v = a[e] + b[e % rows];
-        a[e] = relu ? fmaxf(v, 0.f) : v;
+        const int q = e % rows, j = e / rows;
+        const float v = a[q + ld * j] + b[q];
+        a[q + ld * j] = relu ? fmaxf(v, 0.f) : v;
     }
 }
 
@@ -73,7 +85,8 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
     if (rows_dev) n = (long)(*rows_dev) * mult;
     const long r0 = (long)blockIdx.x * TS;
     if (r0 >= n) return;
-    float *xs = sm, *h1 = xs + nin * TS, *h2 = h1 + H * TS, *o = h2 + H * TS, *dh2 = o + nout * TS;
+    const int lh = act_ld(H), lo = act_ld(nout);
+    float *xs = sm, *h1 = xs + nin * TS, *h2 = h1 + lh * TS, *o = h2 + lh * TS, *dh2 = o + lo * TS;
     const float *W1 = net.par, *b1 = W1 + off_b1(nin, H), *W2 = W1 + off_W2(nin, H), *b2 = W1 + off_b2(nin, H),
                 *W3 = W1 + off_W3(nin, H), *b3 = W1 + off_b3(nin, H, nout);
     const float *xm = net.scale, *xsd = xm + nin, *ym = xsd + nin, *ysd = ym + nout;
@@ -88,23 +101,23 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
         xs[e] = r < 0 ? 0.f : (X[r * nin + f] - xm[f]) / xsd[f];
     }
     __syncthreads();
-    gemm_mfma<false, false>(H, TS, nin, W1, H, xs, nin, h1, H, false);
+    gemm_mfma<false, false>(H, TS, nin, W1, H, xs, nin, h1, lh, false);
     __syncthreads();
-    bias_act(h1, H, b1, true);
+    bias_act(h1, H, lh, b1, true);
     __syncthreads();
-    gemm_mfma<false, false>(H, TS, H, W2, H, h1, H, h2, H, false);
+    gemm_mfma<false, false>(H, TS, H, W2, H, h1, lh, h2, lh, false);
     __syncthreads();
-    bias_act(h2, H, b2, true);
+    bias_act(h2, H, lh, b2, true);
     __syncthreads();
-    gemm_mfma<false, false>(nout, TS, H, W3, nout, h2, H, o, nout, false);
+    gemm_mfma<false, false>(nout, TS, H, W3, nout, h2, lh, o, lo, false);
     __syncthreads();
-    bias_act(o, nout, b3, false);
+    bias_act(o, nout, lo, b3, false);
     __syncthreads();
     if constexpr (!TRAIN) {
         for (int e = threadIdx.x; e < nout * TS; e += MQE_NT) {
             const int q = e % nout, j = e / nout;
             const long r = r0 + j;
-            if (r < n) out[r * nout + q] = o[e] * ysd[q] + ym[q];
+            if (r < n) out[r * nout + q] = o[q + lo * j] * ysd[q] + ym[q];
         }
         return;
     } else {
@@ -116,10 +129,10 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
             const long r = row_of(j);
             float d = 0.f;
             if (r >= 0) {
-                d = o[e] - (Y[r * nout + q] - ym[q]) / ysd[q];
+                d = o[q + lo * j] - (Y[r * nout + q] - ym[q]) / ysd[q];
                 ls += (double)d * d;
             }
-            o[e] = g * d;
+            o[q + lo * j] = g * d;
         }
         __shared__ double red[MQE_WAVES];
         ls = block_sum(ls, red);
@@ -129,34 +142,34 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
         float *gW1 = G, *gb1 = G + off_b1(nin, H), *gW2 = G + off_W2(nin, H), *gb2 = G + off_b2(nin, H),
               *gW3 = G + off_W3(nin, H), *gb3 = G + off_b3(nin, H, nout);
         // layer 3: gW3 = dO h2^T, gb3 = rows of dO, dh2 = W3^T dO masked by h2 > 0
-        gemm_mfma<false, true>(nout, H, TS, o, nout, h2, H, gW3, nout, false);
-        gemm_mfma<true, false>(H, TS, nout, W3, nout, o, nout, dh2, H, false);
+        gemm_mfma<false, true>(nout, H, TS, o, lo, h2, lh, gW3, nout, false);
+        gemm_mfma<true, false>(H, TS, nout, W3, nout, o, lo, dh2, lh, false);
         for (int q = threadIdx.x; q < nout; q += MQE_NT) {
             float s = 0.f;
-            for (int j = 0; j < TS; ++j) s += o[q + nout * j];
+            for (int j = 0; j < TS; ++j) s += o[q + lo * j];
             gb3[q] = s;
         }
         __syncthreads();
-        for (int e = threadIdx.x; e < H * TS; e += MQE_NT)
+        for (int e = threadIdx.x; e < lh * TS; e += MQE_NT)  // (the padding rows are not read)
             if (!(h2[e] > 0.f)) dh2[e] = 0.f;
         __syncthreads();
         // layer 2: gW2 = dh2 h1^T, gb2, dh1 = W2^T dh2 (into h2) masked by h1 > 0
-        gemm_mfma<false, true>(H, H, TS, dh2, H, h1, H, gW2, H, false);
-        gemm_mfma<true, false>(H, TS, H, W2, H, dh2, H, h2, H, false);
+        gemm_mfma<false, true>(H, H, TS, dh2, lh, h1, lh, gW2, H, false);
+        gemm_mfma<true, false>(H, TS, H, W2, H, dh2, lh, h2, lh, false);
         for (int q = threadIdx.x; q < H; q += MQE_NT) {
             float s = 0.f;
-            for (int j = 0; j < TS; ++j) s += dh2[q + H * j];
+            for (int j = 0; j < TS; ++j) s += dh2[q + lh * j];
             gb2[q] = s;
         }
         __syncthreads();
-        for (int e = threadIdx.x; e < H * TS; e += MQE_NT)
+        for (int e = threadIdx.x; e < lh * TS; e += MQE_NT)
             if (!(h1[e] > 0.f)) h2[e] = 0.f;
         __syncthreads();
         // layer 1: gW1 = dh1 xs^T, gb1
-        gemm_mfma<false, true>(H, nin, TS, h2, H, xs, nin, gW1, H, false);
+        gemm_mfma<false, true>(H, nin, TS, h2, lh, xs, nin, gW1, H, false);
         for (int q = threadIdx.x; q < H; q += MQE_NT) {
             float s = 0.f;
-            for (int j = 0; j < TS; ++j) s += h2[q + H * j];
+            for (int j = 0; j < TS; ++j) s += h2[q + lh * j];
             gb1[q] = s;
         }
     }
@@ -164,10 +177,10 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
 
 // Sum of the tile gradients (in a fixed order: wave w of a workgroup takes the
 // tiles congruent to w, the waves' sums are added in their order) and one Adam step.
-// What bounds it: memory, one pass over the tile gradients (22 MB for 16,384 rows
-// at H = 128).  A thread takes one parameter and keeps 16 tiles' loads in flight;
+// What bounds it: memory, one pass over the tile gradients (44 MB for 16,384 rows
+// at H = 128, 8.9 us).  A thread takes one parameter and keeps 16 tiles' loads in flight;
 // one thread per parameter over all tiles in turn, with 85 workgroups, waited for
-// 256 loads one after the other for 60 us: a loss_grad call from 287 to 230 us.
+// 256 loads one after the other for 60 us (at half as many tiles).
 constexpr int SUM_P = 64;  // parameters of a workgroup, one per lane
 __global__ __launch_bounds__(MQE_NT) void adam_kernel(float *par, float *m, float *v, const float *gpart, int ntiles,
                                                       long np, float lr, float b1, float b2, float eps, float c1,
