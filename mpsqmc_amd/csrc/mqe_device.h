@@ -547,8 +547,7 @@ __device__ __forceinline__ void gemm_tiles(int m, int n, int k, const float *A0,
     }
 }
 
-// Single-term products with the original entry points (also used by the
-// proposal network).
+// Single products with operands in LDS or memory (the proposal network's layers).
 template <bool TA, bool TB>
 __device__ __forceinline__ void gemm_mfma(int m, int n, int k, const float *A0, int lda, const float *B0, int ldb,
                                           float *C0, int ldc, bool acc, int nb = 1, long sA = 0, long sB = 0,
