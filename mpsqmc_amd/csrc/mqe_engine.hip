@@ -1290,7 +1290,7 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
     {
         std::vector<int> fill(csptr.begin(), csptr.end());
         for (int c = 0; c < nC; ++c) csidx[fill[second[c]]++] = c;
-        // by first site: the energy sweep picks partners up from left to right
+        // by first site: the energy sweep meets a site's partners in their order along the chain
         for (int k = 0; k < L; ++k)
             std::stable_sort(csidx.begin() + csptr[k], csidx.begin() + csptr[k + 1],
                              [&](int a, int b) { return first[a] < first[b]; });

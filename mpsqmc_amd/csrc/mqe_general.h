@@ -189,8 +189,8 @@ __device__ __forceinline__ void compute_V(const Ctx<T, CH> &C, int j) {
 // Carry four channels (t_k x w_k, ld t_k, contiguous at src) through site k
 // into dst (t_{k+1} x w_{k+1}): dst_ch = sum_s T_k[s]^T src_ch phi_k[s].
 template <typename T, bool CH>
-// nch: the number of channels (4, or 3 for the operator channels of a bond energy).
-__device__ __forceinline__ void carry_channels(const Ctx<T, CH> &C, int k, const T *src, T *dst, int nch = 4) {
+__device__ __forceinline__ void carry_channels(const Ctx<T, CH> &C, int k, const T *src, T *dst) {
+    constexpr int nch = 4;
     const int tk = C.tv[k], tn = C.tv[k + 1], wk = C.wv[k], wn = C.wv[k + 1];
     const T *Tk = C.tsite(k);
     if constexpr (CH) {
@@ -224,6 +224,50 @@ __device__ __forceinline__ void carry_channels(const Ctx<T, CH> &C, int k, const
     // dst_ch = T_k[0]^T Y_ch[0] + T_k[1]^T Y_ch[1], one accumulation chain per output tile
     gemm2<true, false, T>(tn, wn, tk, Tk, Tk + (size_t)tk * tn, tk, Y, Y + (size_t)tk * wn, tk, dst, tn, C.tile, nch, 0,
                           sy, (long)tn * wn);
+    __syncthreads();
+}
+
+// Carry nch channels of a right part (t_{k+1} x w_{k+1}, ld t_{k+1}, contiguous at
+// src) through site k into dst (t_k x w_k): dst_ch = sum_s T_k[s] src_ch phi_k[s]^T.
+template <typename T, bool CH>
+__device__ __forceinline__ void carry_left(const Ctx<T, CH> &C, int k, const T *src, T *dst, int nch) {
+    const int tk = C.tv[k], tn = C.tv[k + 1], wk = C.wv[k], wn = C.wv[k + 1];
+    const T *ph = C.site(k);
+    if constexpr (CH) {
+        constexpr bool TRT = Ctx<T, CH>::TRT;
+        const int ldc = TRT ? tn : tk;
+        const T *TTk = C.tsiteR(k);
+        auto unit = [&](int ch) {
+            ChainOps<T> o;
+            o.A = src + (size_t)ch * tn * wn;
+            o.B[0] = ph;
+            o.B[1] = ph + (size_t)wk * wn;
+            o.C[0] = TTk;
+            o.C[1] = TTk + (size_t)tk * tn;
+            o.D[0] = o.D[1] = dst + (size_t)ch * tk * wk;
+            return o;
+        };
+        if constexpr (sizeof(T) == sizeof(float)) {
+            if (wk >= 32) {
+                chain2<true, TRT, 2, 1>(0, nch, tn, wk, wn, tk, tn, wk, ldc, tk, false, unit);
+                __syncthreads();
+                return;
+            }
+        }
+        chain2_16<true, TRT, 2, 1, T>(0, nch, tn, wk, wn, tk, tn, wk, ldc, tk, false, unit);
+        __syncthreads();
+        return;
+    }
+    T *Y = C.ts + C.sl.Y4;  // Y_ch[s] = src_ch phi_k[s]^T, the two blocks of a channel one after the other
+    const long sy = (long)tn * 2 * wk;
+#pragma nounroll
+    for (int s = 0; s < 2; ++s)
+        gemm_batch<false, true, T>(nch, tn, wk, wn, src, tn, (long)tn * wn, ph + (size_t)s * wk * wn, wk, 0,
+                                   Y + (size_t)s * tn * wk, tn, sy, false, C.tile);
+    __syncthreads();
+    const T *Tk = C.tsite(k);
+    gemm2<false, false, T>(tk, wk, tn, Tk, Tk + (size_t)tk * tn, tk, Y, Y + (size_t)tn * wk, tn, dst, tk, C.tile, nch,
+                           0, sy, (long)tk * wk);
     __syncthreads();
 }
 
@@ -280,23 +324,25 @@ __device__ __forceinline__ void pair_tensor(const Ctx<T, CH> &C, int tb, int wb,
     __syncthreads();
 }
 
-// Bond energy <trial|S_i . S_j|phi> from the three operator channels of site i
-// carried to bond j (c[0] = S^z, c[1] = S^+, c[2] = S^- applied at site i; t_j x
-// w_j, ld t_j) and the blocks V(t', t) of site j:
+// Bond energies <trial|S_i . S_j|phi> of a site j with partners further left take the
+// three operator channels of site j (R[0] = S^z, R[1] = S^-, R[2] = S^+ applied at site
+// j; t x w, ld t, contiguous), carried left to the partner's bond i + 1, and the blocks
+// G(s', s) of site i there:
 // S_i . S_j = S^z S^z + (S^+ S^- + S^- S^+) / 2, with S^z = diag(-1/2, 1/2),
 // S^+ = |1><0|, S^- = |0><1| in the basis ordered by m (OpSz.cpp, OpSx.cpp,
-// OpISy.cpp).  Rout (or nullptr): also writes R_j = V(0,0) + V(1,1) there.
+// OpISy.cpp).
+
+// The channels at site j's own bond from its blocks V(t', t); Rout (or nullptr): also
+// writes R_j = V(0,0) + V(1,1) there.  Ends with a barrier.
 template <typename T, bool CH>
-__device__ __forceinline__ double pair_energy3(const Ctx<T, CH> &C, int tb, int wb, const T *c, T *Rout = nullptr) {
+__device__ __forceinline__ void operator_channels(const Ctx<T, CH> &C, int tb, int wb, T *R, T *Rout) {
     const T *V = C.ts + C.sl.V;
-    const size_t bs = (size_t)tb * wb;
-    const T *V00 = V, *V01 = V + bs, *V10 = V + 2 * bs, *V11 = V + 3 * bs;  // V(t', t) at t' 2 bs + t bs
-    double acc = 0.0;
-    const int n = (int)bs;
-    // two elements of a thread per pass, loads before the store to Rout (as in
+    const int n = tb * wb;
+    const T *V00 = V, *V01 = V + n, *V10 = V + 2 * (size_t)n, *V11 = V + 3 * (size_t)n;  // V(t', t) at t' 2 n + t n
+    // two elements of a thread per pass, loads before the stores (as in
     // pair_tensor; the clamped second index is skipped below)
     for (int e0 = threadIdx.x; e0 < n; e0 += 2 * MQE_NT) {
-        T v00[2], v11[2], v01[2], v10[2], cz[2], cp[2], cm[2];
+        T v00[2], v11[2], v01[2], v10[2];
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const int e = min(e0 + u * MQE_NT, n - 1);
@@ -304,21 +350,37 @@ __device__ __forceinline__ double pair_energy3(const Ctx<T, CH> &C, int tb, int 
             v11[u] = V11[e];
             v01[u] = V01[e];
             v10[u] = V10[e];
-            cz[u] = c[e];
-            cp[u] = c[bs + e];
-            cm[u] = c[2 * bs + e];
         }
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const int e = e0 + u * MQE_NT;
             if (e < n) {
-                acc += (double)cz[u] * (0.5 * ((double)v11[u] - (double)v00[u])) +
-                       0.5 * ((double)cp[u] * (double)v01[u] + (double)cm[u] * (double)v10[u]);
+                R[e] = (T)0.5 * (v11[u] - v00[u]);
+                R[n + e] = v01[u];
+                R[2 * (size_t)n + e] = v10[u];
                 if (Rout) Rout[e] = v00[u] + v11[u];
             }
         }
     }
-    return block_sum(acc, C.red);
+    __syncthreads();
+}
+
+// This thread's part of the bond energy of (i, j): the channels R at bond i + 1 with
+// the blocks G(s', s) of site i in the G scratch (block at s' t + s 2 t w, ld 2 t).
+template <typename T, bool CH>
+__device__ __forceinline__ double pair_energy_part(const Ctx<T, CH> &C, int tb, int wb, const T *R) {
+    const T *G = C.ts + C.sl.G;
+    const int n = tb * wb;
+    const size_t os = (size_t)wb * 2 * tb;
+    double acc = 0.0;
+    for (int e = threadIdx.x; e < n; e += MQE_NT) {
+        const int a = e % tb, b = e / tb;
+        const size_t o = a + (size_t)2 * tb * b;
+        const T g00 = G[o], g01 = G[o + os], g10 = G[o + tb], g11 = G[o + tb + os];
+        const T rz = R[e], rm = R[n + e], rp = R[2 * (size_t)n + e];
+        acc += 0.5 * (((double)g11 - (double)g00) * (double)rz + (double)g10 * (double)rm + (double)g01 * (double)rp);
+    }
+    return acc;
 }
 
 // The four blocks G(s', s) of site `first` carried to the left of site `bond`
@@ -764,47 +826,32 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
             etot += S.Jc[c] * e;
         }
         if (nq > 0) {
-            // long range: only sum_i J_ik S_i . S_k is needed: the operator channels S^z, S^+, S^-
-            // of site i (ch = 2 s' + s: S^z = (G(1,1) - G(0,0)) / 2, S^+ = G(1,0),
-            // S^- = G(0,1)) times J_ik start at the leftmost partner of k, take in
-            // each further one on their way right, and meet V once at bond k (the FP32
-            // sum costs nothing: relative error of the energy of 64 walkers near the 4x4
-            // torus' trial at D = 20 against FP64 2.0e-7 either way)
+            // long range: the three operator channels of site k start at its bond and
+            // go left once for all its partners, from the nearest to the farthest; each
+            // coupling meets the blocks G of its own first site and is summed, times J,
+            // in FP64 (adding J S_i of the partners up in one set of FP32 channels
+            // instead rounds every coupling to the largest of them; a step of the 6x6
+            // snake at D = 128, 256 walkers: 130 ms that way, 122 ms this way, of a
+            // 15-site ring at D = 20, 200 walkers: 1317 and 1329 us)
             T *A = C.ts + C.sl.GcA, *B = C.ts + C.sl.GcB;
-            int bond = -1;
-            for (int q = q0; q <= q0 + nq; ++q) {
-                const int c = q < q0 + nq ? uni(S.cs_idx[q]) : 0, i = q < q0 + nq ? uni(S.first[c]) : k - 1;
+            operator_channels(C, C.tv[k], C.wv[k], A, r_pending ? C.Rk(k) : nullptr);
+            double ep = 0.0;
+            int bond = k;
+            for (int q = q0 + nq - 1; q >= q0; --q) {
+                const int c = uni(S.cs_idx[q]), i = uni(S.first[c]);
                 const int tn = C.tv[i + 1], wn = C.wv[i + 1];
-                T *G = C.ts + C.sl.G;
-                if (q < q0 + nq) {
-                    if constexpr (CH) {
-                        issue_G(C, i, C.Lk(i), G, 2 * tn, tn, (long)wn * 2 * tn, 0);
-                        if (bond < 0 || bond > i) __syncthreads();
-                    } else {
-                        compute_G(C, i, C.Lk(i));
-                    }
-                }
-                const bool fresh = bond < 0;
-                for (int kk = fresh ? i + 1 : bond; kk <= i; ++kk) {
-                    carry_channels(C, kk, A, B, 3);
+                // (i <= k - 2 and the partners differ: at least one carry, whose
+                // barrier covers G)
+                if constexpr (CH) issue_G(C, i, C.Lk(i), C.ts + C.sl.G, 2 * tn, tn, (long)wn * 2 * tn, 0);
+                else compute_G(C, i, C.Lk(i));
+                for (; bond > i + 1; --bond) {
+                    carry_left(C, bond - 1, A, B, 3);
                     T *t = A; A = B; B = t;
                 }
-                bond = i + 1;
-                if (q == q0 + nq) break;
-                const int nb = tn * wn;
-                const double J = S.Jc[c];
-                for (int e = threadIdx.x; e < nb; e += MQE_NT) {
-                    const int a = e % tn, be = e / tn;
-                    const size_t o = a + (size_t)2 * tn * be, os = (size_t)wn * 2 * tn;
-                    const T g00 = G[o], g01 = G[o + os], g10 = G[o + tn], g11 = G[o + tn + os];
-                    const double z = 0.5 * J * ((double)g11 - (double)g00), pl = J * g10, mi = J * g01;
-                    A[e] = (T)(fresh ? z : (double)A[e] + z);
-                    A[nb + e] = (T)(fresh ? pl : (double)A[nb + e] + pl);
-                    A[2 * nb + e] = (T)(fresh ? mi : (double)A[2 * nb + e] + mi);
-                }
-                __syncthreads();
+                ep += S.Jc[c] * pair_energy_part(C, tn, wn, A);
+                if (q > q0) __syncthreads();  // G is formed anew
             }
-            etot += pair_energy3(C, C.tv[k], C.wv[k], A, r_pending ? C.Rk(k) : nullptr);
+            etot += block_sum(ep, C.red);
         }
         if (S.h != 0.0) {
             // <trial|S^z_k|phi> = sum_t sz[t] <L'_k, V(t,t)>, L'_k the current-gauge left env
