@@ -1108,6 +1108,21 @@ __device__ __forceinline__ double recip_d(double x) {
     return fma(r * e, 1.0 + e, r);
 }
 
+// Binary exponent of a column held by G lanes (the sum of its magnitudes; 0 for a
+// column of zeros or one that is not finite).
+template <int G, int NE>
+__device__ __forceinline__ int column_exponent(const double (&a)[NE]) {
+    double s = 0.0;
+#pragma unroll
+    for (int t = 0; t < NE; ++t) s += fabs(a[t]);
+    return __builtin_amdgcn_frexp_exp(lanes_sum<G>(s));
+}
+template <int NE>
+__device__ __forceinline__ void scale_column(double (&a)[NE], int e) {
+#pragma unroll
+    for (int t = 0; t < NE; ++t) a[t] = __builtin_amdgcn_ldexp(a[t], e);
+}
+
 // ---------------------------------------------------------------------------
 // The same factorisation with every column in registers: LPC lanes own a column
 // (lane ln its rows ln + LPC t, t < NE), so m <= LPC NE and n <= threads / LPC.
@@ -1120,6 +1135,11 @@ __device__ __forceinline__ double recip_d(double x) {
 // put_r(r, c, x): R(r, c) for r <= c, after the last barrier (V may be
 // overwritten there if want_q is false); want_q: put_q(r, c, x) gets Q, after a
 // barrier past the last read of V.  Ends without a barrier.
+// SCALE: every column is brought to unit magnitude by a power of two first and its
+// column of R back afterwards (exact; the column of Q is the same).  The unscaled v
+// and n2 hold squares, so without it a column below 1e-145 was left as it is: needed
+// for FP64 elements, which can be that small, not for the squares of FP32 ones.
+// What is left out then is below 1e-145 of its column.
 // What bounds it: the chain of one column (LDS read, dot products, group sums,
 // root and reciprocal, update, LDS write, barrier), which nothing overlaps within
 // a walker.  So rows past m are zeros instead of bounds checks, groups that are
@@ -1128,7 +1148,7 @@ __device__ __forceinline__ double recip_d(double x) {
 // one sweep over the 31 inner sites of a D = 32 chain added 1258 us to a step,
 // now 681 us.
 // ---------------------------------------------------------------------------
-template <int LPC, int NE, class Load, class PutR, class PutQ>
+template <int LPC, int NE, bool SCALE = false, class Load, class PutR, class PutQ>
 __device__ __forceinline__ void qr_regs(int m, int n, double *V, double *tau, bool want_q, Load load, PutR put_r,
                                         PutQ put_q) {
     constexpr int LDV = LPC * NE;
@@ -1141,6 +1161,8 @@ __device__ __forceinline__ void qr_regs(int m, int n, double *V, double *tau, bo
         a[t] = r < m && g < n ? load(r, g) : 0.0;
         x[t] = 0.0;
     }
+    const int ex = SCALE ? column_exponent<LPC>(a) : 0;
+    if (SCALE) scale_column(a, -ex);
     __syncthreads();  // V may overlay what load() reads
     double *vg = V + LDV * g + ln;
     if (g == 0) {
@@ -1172,7 +1194,7 @@ __device__ __forceinline__ void qr_regs(int m, int n, double *V, double *tau, bo
             s = lanes_sum<LPC>(s);
             aj = lanes_sum<LPC>(aj);
             const double n2 = fma(alpha, alpha, ss), nrm = n2 * rsqrt_d(n2), d = nrm + fabs(alpha);
-            const bool on = ss > 0.0 && n2 > 1e-290;  // (the squares of anything smaller are lost to underflow)
+            const bool on = ss > 0.0 && n2 > 1e-290;  // (the products of anything smaller are lost to underflow)
             const double vjj = on ? copysign(d, alpha) : 1.0, tj = on ? recip_d(nrm * d) : 0.0;
             const double f = g >= j ? tj * fma(vjj, aj, s) : 0.0;
 #pragma unroll
@@ -1192,7 +1214,7 @@ __device__ __forceinline__ void qr_regs(int m, int n, double *V, double *tau, bo
 #pragma unroll
         for (int t = 0; t < NE; ++t) {
             const int r = ln + LPC * t;
-            if (r <= g) put_r(r, g, a[t]);
+            if (r <= g) put_r(r, g, SCALE ? __builtin_amdgcn_ldexp(a[t], ex) : a[t]);
         }
     }
     if (!want_q) return;
@@ -1240,11 +1262,11 @@ __device__ __forceinline__ void qr_regs(int m, int n, double *V, double *tau, bo
 // 128 x 64.  qr_doubles: LDS of V and tau for any matrix of at most 2 D x D.
 constexpr int QR_REGS_M = 128, QR_REGS_N = 64;
 __host__ __device__ constexpr long qr_doubles(int D) { return (D <= 32 ? 64L : 128L) * D + D; }
-template <class Load, class PutR, class PutQ>
+template <bool SCALE, class Load, class PutR, class PutQ>
 __device__ __forceinline__ void qr_in_regs(int m, int n, double *V, double *tau, bool want_q, Load load, PutR put_r,
                                            PutQ put_q) {
-    if (m <= 64 && n <= 32) qr_regs<8, 8>(m, n, V, tau, want_q, load, put_r, put_q);
-    else qr_regs<4, 32>(m, n, V, tau, want_q, load, put_r, put_q);
+    if (m <= 64 && n <= 32) qr_regs<8, 8, SCALE>(m, n, V, tau, want_q, load, put_r, put_q);
+    else qr_regs<4, 32, SCALE>(m, n, V, tau, want_q, load, put_r, put_q);
 }
 
 // ---------------------------------------------------------------------------
@@ -1264,7 +1286,7 @@ constexpr int QR_PANEL = 32, QR_PANELS_M = 256, QR_PANELS_N = 128;
 __host__ __device__ constexpr long panel_doubles(int n) {
     return (long)QR_PANELS_M * QR_PANEL * ((n + QR_PANEL - 1) / QR_PANEL);
 }
-template <class Load, class PutR, class PutQ>
+template <bool SCALE, class Load, class PutR, class PutQ>
 __device__ __forceinline__ void qr_panels(int m, int n, double *V, double *tau, double *W, Load load, PutR put_r,
                                           PutQ put_q) {
     constexpr int LPC = 8, NE = 32, LDV = QR_PANELS_M, PC = QR_PANEL, BLOCK = LDV * PC;
@@ -1313,6 +1335,8 @@ __device__ __forceinline__ void qr_panels(int m, int n, double *V, double *tau, 
             const int r = ln + LPC * t;
             a[t] = r < m && g < nc ? load(r, base + g) : 0.0;
         }
+        const int ex = SCALE ? column_exponent<LPC>(a) : 0;
+        if (SCALE) scale_column(a, -ex);
         for (int q = 0; q < c; ++q) {
             if (q != c - 1 || c > 1) fetch(q);  // panel 0 is still in LDS when panel 1 needs it
             apply(PC * q, PC, 0, 1, false);
@@ -1372,7 +1396,7 @@ __device__ __forceinline__ void qr_panels(int m, int n, double *V, double *tau, 
 #pragma unroll
             for (int t = 0; t < NE; ++t) {
                 const int r = ln + LPC * t;
-                if (r <= base + g) put_r(r, base + g, a[t]);
+                if (r <= base + g) put_r(r, base + g, SCALE ? __builtin_amdgcn_ldexp(a[t], ex) : a[t]);
             }
         }
         __syncthreads();

@@ -167,8 +167,8 @@ __device__ __forceinline__ void compress_bond(const Pool &P, T *phi, int *wv, in
     // R of the QR of a rows x cols matrix (rows >= cols) given by load, to Y (ld cols)
     auto r_factor = [&](int rows, int cols, auto load) {
         if constexpr (SM) {
-            qr_in_regs(rows, cols, Y, sig, false, load, [&](int i, int j, double x) { Y[i + (size_t)cols * j] = x; },
-                       nothing);
+            qr_in_regs<sizeof(T) == 8>(rows, cols, Y, sig, false, load,
+                                       [&](int i, int j, double x) { Y[i + (size_t)cols * j] = x; }, nothing);
             __syncthreads();
         } else {  // in X's place (the caller fills X afterwards), R to Y
             for (int e = tid; e < rows * cols; e += MQE_NT) X[e] = load(e % rows, e / rows);
@@ -206,9 +206,9 @@ __device__ __forceinline__ void compress_bond(const Pool &P, T *phi, int *wv, in
     bool basis_only = false;
     if constexpr (SM) {
         if (rc <= m && rc <= D) {
-            qr_in_regs(m, rc, X, sig, true, [&](int i, int j) { return X[i + (size_t)ldx * j]; },
-                       [&](int i, int j, double x) { Y[i + (size_t)rc * j] = x; },
-                       [&](int i, int j, double x) { X[i + (size_t)ldx * j] = x; });
+            qr_in_regs<sizeof(T) == 8>(m, rc, X, sig, true, [&](int i, int j) { return X[i + (size_t)ldx * j]; },
+                                       [&](int i, int j, double x) { Y[i + (size_t)rc * j] = x; },
+                                       [&](int i, int j, double x) { X[i + (size_t)ldx * j] = x; });
             __syncthreads();
             // ten times the cut: the bound's own rounding cannot matter
             basis_only = least_singular_bound(Y, rc, Y + (size_t)rc * rc, red) > 10 * SCHMIDT_CUT;

@@ -653,9 +653,9 @@ __device__ __noinline__ void lq_factor(T *ph_, T *LM_, double *AQ_, double *RQ_,
     auto put_q = [&](int r, int c, double x) { ph[c + (size_t)wk * r] = (T)x; };
     const bool fits = nq > 0 && n <= m;
     if (fits && m <= QR_REGS_M && n <= QR_REGS_N && nq >= (m <= 64 && n <= 32 ? 65 : 129) * n) {
-        qr_in_regs(m, n, qlds_dyn + n, qlds_dyn, true, load, put_r, put_q);
+        qr_in_regs<sizeof(T) == 8>(m, n, qlds_dyn + n, qlds_dyn, true, load, put_r, put_q);
     } else if (PANELS && fits && m <= QR_PANELS_M && n <= QR_PANELS_N && nq >= QR_PANELS_M * QR_PANEL + n) {
-        qr_panels(m, n, qlds_dyn + n, qlds_dyn, AQ, load, put_r, put_q);
+        qr_panels<sizeof(T) == 8>(m, n, qlds_dyn + n, qlds_dyn, AQ, load, put_r, put_q);
     } else {
         double *R = (double *)uni((long)RQ_);
         double *tau = nq > 0 ? qlds_dyn : (double *)uni((long)TAU_);
