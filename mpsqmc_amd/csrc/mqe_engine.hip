@@ -772,6 +772,10 @@ using namespace mqe;
         }                                                                                    \
     } while (0)
 
+// floats of the staging buffer of an upload (a synchronous copy costs about 10 us
+// whatever its size up to here)
+constexpr long STAGE = 32768;
+
 struct mqe_engine {
     mqe_params p;
     int L = 0, nC = 0, Ng = 0, gdim = 0, Dt = 0, Dw = 0;
@@ -781,6 +785,7 @@ struct mqe_engine {
     float *d_trialT = nullptr;  // chained general kernel: every T_k[s] transposed
     bool chained = false;       // the general kernel with chained products (bonds <= 64)
     hipStream_t stream = nullptr;
+    std::vector<float> stage;  // FP32: host staging of mqe_overlaps
     std::vector<int> tvd, wmax;
     std::vector<long> toff, woff, eoff, moff;
     long wflat = 0, eflat = 0, scratch_bytes = 0;
@@ -1096,8 +1101,9 @@ int overlaps_in_workspace(mqe_engine *e, const mqe_mps *other, double *out, char
         return MQE_ECAPACITY;
     }
     const int chunk = (int)std::min<size_t>((size_t)std::max(n, 1), ((size_t)ws_bytes - pl.off_ws) / pl.per_walker);
-    // stage the other MPS in the engine's precision, its dims and offsets
-    // (fixed-size host buffers: this path allocates nothing on host or device)
+    // stage the other MPS in the engine's precision, its dims and offsets (the
+    // engine's own host buffer: this path allocates nothing on host or device, and
+    // its caller's stack may be a small one)
     long off[MQE_MAXL];
     long t = 0;
     for (int k = 0; k < L; ++k) {
@@ -1105,10 +1111,9 @@ int overlaps_in_workspace(mqe_engine *e, const mqe_mps *other, double *out, char
         t += (long)other->vd[k] * other->vd[k + 1] * 2;
     }
     if (e->fp32) {
-        constexpr long CHUNK = 32768;  // a synchronous copy costs about 10 us whatever its size here
-        float tmp[CHUNK];
-        for (long i0 = 0; i0 < pl.tot; i0 += CHUNK) {
-            const long m = std::min(CHUNK, pl.tot - i0);
+        float *tmp = e->stage.data();
+        for (long i0 = 0; i0 < pl.tot; i0 += STAGE) {
+            const long m = std::min(STAGE, pl.tot - i0);
             for (long i = 0; i < m; ++i) tmp[i] = (float)other->data[i0 + i];
             HIPCHK(hipMemcpy(ws + sizeof(float) * i0, tmp, sizeof(float) * m, hipMemcpyHostToDevice));
         }
@@ -1164,6 +1169,7 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
     e->Ng = n_grid;
     e->gdim = grid_dim;
     e->fp32 = p->precision == MQE_PREC_FP32;
+    if (e->fp32) e->stage.resize(STAGE);
     e->tvd.assign(trial->vd, trial->vd + L + 1);
     e->Dt = *std::max_element(e->tvd.begin(), e->tvd.end());
     e->wmax.resize(L + 1);
