@@ -140,9 +140,10 @@ int mqe_compress_walkers(mqe_engine *e, const int *targets);
  * chosen per walker by its bond bucket (largest bond 1-16, 17-32, ..., > 112)
  * from an 8-entry table: tiles[bucket] in {16, 32, 64}.  mqe_create takes the
  * table tuned for the engine's key (L, couplings, trial and walker bonds,
- * precision) from the cache file ($MQE_TUNE_CACHE, else
- * ~/.cache/mqe_tiles.txt) when it has one.  Results do not depend on the
- * table beyond FP32 rounding; FP64 engines and the tile path ignore it. */
+ * precision, and the version of the products that it was timed on) from the
+ * cache file ($MQE_TUNE_CACHE, else ~/.cache/mqe_tiles.txt) when it has one.
+ * Results do not depend on the table beyond FP32 rounding; FP64 engines and
+ * the tile path ignore it. */
 int mqe_get_tiles(mqe_engine *e, int *tiles);
 int mqe_set_tiles(mqe_engine *e, const int *tiles);
 /* Time `reps` propagations of the current population with each candidate

@@ -786,6 +786,7 @@ struct mqe_engine {
     bool chained = false;       // the general kernel with chained products (bonds <= 64)
     hipStream_t stream = nullptr;
     std::vector<float> stage;  // FP32: host staging of mqe_overlaps
+    unsigned long long pair_hash = 0;  // of the coupled pairs (key of the tile table)
     std::vector<int> tvd, wmax;
     std::vector<long> toff, woff, eoff, moff;
     long wflat = 0, eflat = 0, scratch_bytes = 0;
@@ -1166,6 +1167,9 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
     e->p = *p;
     e->L = L;
     e->nC = n_couplings;
+    e->pair_hash = 1469598103934665603ull;  // FNV-1a
+    for (int c = 0; c < n_couplings; ++c)
+        for (int x : {first[c], second[c]}) e->pair_hash = (e->pair_hash ^ (unsigned)x) * 1099511628211ull;
     e->Ng = n_grid;
     e->gdim = grid_dim;
     e->fp32 = p->precision == MQE_PREC_FP32;
@@ -1722,11 +1726,20 @@ int mqe_kernel_path(mqe_engine *e) { return (e && e->tile32) ? 1 : 0; }
 }  // extern "C"
 
 // ---- tile-shape autotuner -----------------------------------------------------
+// Version of the products that the tables are tuned on.  A table is worth nothing on
+// other kernels (one tuned before the products above bonds of 64 were rewritten set
+// them back to 32 x 32 tiles: 141 instead of 130 ms a step of the 6x6 snake at
+// D = 128): raise it with every change of gemm_tiles_buf, the chained products, the
+// choice between them or the default table.
+constexpr int TILE_TABLE_VERSION = 2;
+
 // Key of the tuned table: the product shapes depend on the trial and walker
-// bonds, the chain length, the couplings and the precision.
+// bonds, the chain length, the couplings (which pairs: a hash) and the precision, their
+// times on the kernel that runs them.
 static std::string tune_key(const mqe_engine *e) {
     char b[160];
-    snprintf(b, sizeof(b), "L%d_nC%d_Dt%d_Dw%d_d%d_%s", e->L, e->nC, e->Dt, e->Dw, e->p.d, e->fp32 ? "fp32" : "fp64");
+    snprintf(b, sizeof(b), "v%d_L%d_nC%d_%016llx_Dt%d_Dw%d_d%d_%s%s", TILE_TABLE_VERSION, e->L, e->nC, e->pair_hash,
+             e->Dt, e->Dw, e->p.d, e->fp32 ? "fp32" : "fp64", e->chained ? "_chained" : "");
     return b;
 }
 
