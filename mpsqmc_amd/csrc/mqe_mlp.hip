@@ -12,7 +12,8 @@
 // MFMA GEMM (v_mfma_f32_32x32x2f32) with the weights read from global memory
 // (80 KB at H = 128, L2-resident).  Training computes forward and backward of a
 // tile and writes the tile's gradient to its own slot; the Adam kernel sums the
-// slots in a fixed order (deterministic) and updates the parameters.
+// slots in a fixed order (deterministic) and updates the parameters.  More rows than
+// there are slots for take turns.
 //
 // Parameter layout (column-major): W1 [H x n_in], b1 [H], W2 [H x H], b2 [H],
 // W3 [n_out x H], b3 [n_out].  Inputs are standardised with (x - x_mean) /
@@ -39,6 +40,10 @@ namespace mlp {
 // 16,384 rows 88 -> 79 us; with the padded blocks below 80 and 71 us.
 constexpr int TS = 32;
 constexpr int MAX_IN = 32, MAX_H = 128, MAX_OUT = 32;
+// Gradient slots, and so the tiles of one training launch: twice as many as
+// workgroups that fit the chip (two a CU at H = 128).  90 MB at H = 128 whatever the
+// number of rows; a slot for every tile took 2.7 KB a row.
+constexpr long SLOTS = 1024;
 
 struct Net {
     int nin, H, nout;
@@ -74,16 +79,16 @@ __device__ __forceinline__ void bias_act(float *a, int rows, int ld, const float
     }
 }
 
-// Rows of the tile: r < n valid.  perm (optional) maps tile rows to data rows.
+// Tiles of the rows from `first` on: r < n valid.  perm (optional) maps tile rows to data rows.
 // rows_dev (optional): the row count is *rows_dev * mult (device-side count).
 template <bool TRAIN>
-__global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, const float *Y, long n,
+__global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, const float *Y, long first, long n,
                                                       const int *rows_dev, int mult, const int *perm, float *out,
                                                       float *gpart, double *loss) {
     extern __shared__ float sm[];
     const int nin = net.nin, H = net.H, nout = net.nout;
     if (rows_dev) n = (long)(*rows_dev) * mult;
-    const long r0 = (long)blockIdx.x * TS;
+    const long r0 = first + (long)blockIdx.x * TS;
     if (r0 >= n) return;
     const int lh = act_ld(H), lo = act_ld(nout);
     float *xs = sm, *h1 = xs + nin * TS, *h2 = h1 + lh * TS, *o = h2 + lh * TS, *dh2 = o + lo * TS;
@@ -177,6 +182,7 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
 
 // Sum of the tile gradients (in a fixed order: wave w of a workgroup takes the
 // tiles congruent to w, the waves' sums are added in their order) and one Adam step.
+// more: grad_out holds the sum over the rows before these.  step: take the Adam step, else write the sum there.
 // What bounds it: memory, one pass over the tile gradients (44 MB for 16,384 rows
 // at H = 128, 8.9 us).  A thread takes one parameter and keeps 16 tiles' loads in flight;
 // one thread per parameter over all tiles in turn, with 85 workgroups, waited for
@@ -184,7 +190,7 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
 constexpr int SUM_P = 64;  // parameters of a workgroup, one per lane
 __global__ __launch_bounds__(MQE_NT) void adam_kernel(float *par, float *m, float *v, const float *gpart, int ntiles,
                                                       long np, float lr, float b1, float b2, float eps, float c1,
-                                                      float c2, float *grad_out) {
+                                                      float c2, float *grad_out, bool more, bool step) {
     __shared__ float part[MQE_WAVES][SUM_P];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const long p = (long)blockIdx.x * SUM_P + lane;
@@ -204,10 +210,10 @@ __global__ __launch_bounds__(MQE_NT) void adam_kernel(float *par, float *m, floa
     part[w][lane] = g;
     __syncthreads();
     if (w != 0 || p >= np) return;
-    g = 0.f;
+    g = more ? grad_out[p] : 0.f;
 #pragma unroll
     for (int q = 0; q < MQE_WAVES; ++q) g += part[q][lane];
-    if (grad_out) {
+    if (!step) {
         grad_out[p] = g;
         return;
     }
@@ -271,6 +277,7 @@ int ensure_gpart(mqe_mlp *m, long tiles) {
     if (tiles <= m->gpart_tiles) return MQE_OK;
     if (m->d_gpart) MCHK(hipFree(m->d_gpart));
     m->d_gpart = nullptr;
+    m->gpart_tiles = 0;
     MCHK(hipMalloc((void **)&m->d_gpart, sizeof(float) * (size_t)tiles * m->np));
     m->gpart_tiles = tiles;
     return MQE_OK;
@@ -295,15 +302,29 @@ int set_lds(mqe_mlp *m) {
     return MQE_OK;
 }
 
-// loss and tile gradients of rows [0, n) (through perm when given) into d_gpart
-int grad_pass(mqe_mlp *m, const float *dX, const float *dY, long n, const int *dperm) {
-    const long tiles = (n + mlp::TS - 1) / mlp::TS;
-    int r = ensure_gpart(m, tiles);
+// the constants of one Adam step
+struct AdamStep {
+    float lr = 0.f, b1 = 0.f, b2 = 0.f, eps = 0.f, c1 = 1.f, c2 = 1.f;
+};
+
+// loss and gradient of rows [0, n) (through perm when given), SLOTS tiles at a time; then
+// the step, or the gradient to d_grad
+int grad_pass(mqe_mlp *m, const float *dX, const float *dY, long n, const int *dperm, const AdamStep *step) {
+    int r = ensure_gpart(m, std::min((n + mlp::TS - 1) / mlp::TS, mlp::SLOTS));
     if (r) return r;
-    hipLaunchKernelGGL(mlp::tile_kernel<true>, dim3((unsigned)tiles), dim3(MQE_NT),
-                       mlp::lds_bytes(m->nin, m->H, m->nout, true), m->stream, m->net(), dX, dY, n,
-                       (const int *)nullptr, 0, dperm, (float *)nullptr, m->d_gpart, m->d_loss);
-    MCHK(hipGetLastError());
+    for (long first = 0; first < n; first += mlp::SLOTS * mlp::TS) {
+        const long tiles = std::min((n - first + mlp::TS - 1) / mlp::TS, mlp::SLOTS);
+        const bool last = first + mlp::SLOTS * mlp::TS >= n;
+        hipLaunchKernelGGL(mlp::tile_kernel<true>, dim3((unsigned)tiles), dim3(MQE_NT),
+                           mlp::lds_bytes(m->nin, m->H, m->nout, true), m->stream, m->net(), dX, dY, first, n,
+                           (const int *)nullptr, 0, dperm, (float *)nullptr, m->d_gpart, m->d_loss);
+        MCHK(hipGetLastError());
+        const AdamStep a = step ? *step : AdamStep();
+        hipLaunchKernelGGL(mlp::adam_kernel, dim3((unsigned)((m->np + mlp::SUM_P - 1) / mlp::SUM_P)), dim3(MQE_NT), 0,
+                           m->stream, m->d_par, m->d_m, m->d_v, m->d_gpart, (int)tiles, m->np, a.lr, a.b1, a.b2, a.eps,
+                           a.c1, a.c2, m->d_grad, first > 0, last && step);
+        MCHK(hipGetLastError());
+    }
     return MQE_OK;
 }
 
@@ -318,7 +339,7 @@ int mlp_forward_device(mqe_mlp *m, const float *dX, long max_rows, const int *ro
     const long tiles = (max_rows + mlp::TS - 1) / mlp::TS;
     if (tiles <= 0) return MQE_OK;
     hipLaunchKernelGGL(mlp::tile_kernel<false>, dim3((unsigned)tiles), dim3(MQE_NT),
-                       mlp::lds_bytes(m->nin, m->H, m->nout, false), s, m->net(), dX, (const float *)nullptr,
+                       mlp::lds_bytes(m->nin, m->H, m->nout, false), s, m->net(), dX, (const float *)nullptr, 0L,
                        max_rows, rows_dev, mult, (const int *)nullptr, dY, (float *)nullptr, (double *)nullptr);
     MCHK(hipGetLastError());
     return MQE_OK;
@@ -365,15 +386,11 @@ int mlp_fit_device(mqe_mlp *m, const float *dX, const float *dY, long n, int epo
         MCHK(hipMemsetAsync(m->d_loss, 0, sizeof(double), s));
         for (long r0 = 0; r0 < n; r0 += batch) {
             const long nb = std::min((long)batch, n - r0);
-            int r = grad_pass(m, dX, dY, nb, m->d_perm + r0);
+            const float t = (float)(m->adam_t + 1);
+            const AdamStep step{(float)lr, b1, b2, eps, 1.f - powf(b1, t), 1.f - powf(b2, t)};
+            const int r = grad_pass(m, dX, dY, nb, m->d_perm + r0, &step);
             if (r) return r;
             ++m->adam_t;
-            const float c1 = 1.f - powf(b1, (float)m->adam_t), c2 = 1.f - powf(b2, (float)m->adam_t);
-            const int tiles = (int)((nb + mlp::TS - 1) / mlp::TS);
-            hipLaunchKernelGGL(mlp::adam_kernel, dim3((unsigned)((m->np + mlp::SUM_P - 1) / mlp::SUM_P)),
-                               dim3(MQE_NT), 0, s, m->d_par, m->d_m, m->d_v, m->d_gpart, tiles, m->np, (float)lr, b1,
-                               b2, eps, c1, c2, (float *)nullptr);
-            MCHK(hipGetLastError());
         }
         // the loss accumulated over the epoch's minibatches, per standardised output
         double lsum = 0.0;
@@ -517,14 +534,8 @@ int mqe_mlp_loss_grad(mqe_mlp *m, int n, const float *X, const float *Y, double 
     MCHK(hipMemcpyAsync(m->d_X, X, sizeof(float) * (size_t)n * m->nin, hipMemcpyHostToDevice, m->stream));
     MCHK(hipMemcpyAsync(m->d_Y, Y, sizeof(float) * (size_t)n * m->nout, hipMemcpyHostToDevice, m->stream));
     MCHK(hipMemsetAsync(m->d_loss, 0, sizeof(double), m->stream));
-    r = grad_pass(m, m->d_X, m->d_Y, n, nullptr);
+    r = grad_pass(m, m->d_X, m->d_Y, n, nullptr, nullptr);
     if (r) return r;
-    const int tiles = (int)((n + mlp::TS - 1) / mlp::TS);
-    // grad_out mode of the Adam kernel: the summed gradient, no update
-    hipLaunchKernelGGL(mlp::adam_kernel, dim3((unsigned)((m->np + mlp::SUM_P - 1) / mlp::SUM_P)), dim3(MQE_NT), 0,
-                       m->stream, m->d_par, m->d_m, m->d_v, m->d_gpart, tiles, m->np, 0.f, 0.f, 0.f, 0.f, 1.f, 1.f,
-                       m->d_grad);
-    MCHK(hipGetLastError());
     double ls = 0.0;
     MCHK(hipMemcpyAsync(&ls, m->d_loss, sizeof(double), hipMemcpyDeviceToHost, m->stream));
     if (grad) MCHK(hipMemcpyAsync(grad, m->d_grad, sizeof(float) * m->np, hipMemcpyDeviceToHost, m->stream));
