@@ -10,6 +10,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #define MQE_NT 256
 #define MQE_WAVES (MQE_NT / 64)
 
@@ -152,51 +154,15 @@ __device__ __forceinline__ void block_inclusive_scan(int n, const double *x, dou
 }
 
 // ---------------------------------------------------------------------------
-// FP32 GEMM on the matrix cores: C(m x n) = sum_{s < nseg} op(A_s) op(B_s)
-// (nseg = 1 or 2 terms of one shape and leading dimensions), for nb products
-// at once (A_s + b sA and so on), whole workgroup.  The output is cut into
-// tiles, one wave per tile at a time; the tiles of all nb products are shared
-// among the four waves.  Each tile is a chain of MFMAs over the k slices of
-// its terms.  A lane's operand values of a slice are one run along k, loaded
-// straight into the MFMA operand registers without predication: rows and
-// columns beyond the matrix are clamped to its last row / column (they only
-// feed output elements that are not stored), so the wait for a slice's data
-// sits right before its MFMAs, and the loads of the wave's next slice (of this
-// tile or the first of its next tile) are issued before the MFMAs of the
-// current one.  k not a multiple of the slice depth (16) takes a predicated
-// path with zeros outside the matrices.  acc: C += instead of C =.
+// FP32 GEMM on the matrix cores, whole workgroup.  The output is cut into
+// tiles, one wave per tile at a time, each a chain of MFMAs over the k slices.
+// A lane's operand values of a slice are one run along k, loaded straight into
+// the MFMA operand registers without predication: rows and columns beyond the
+// matrix are clamped to its last row / column (they only feed output elements
+// that are not stored), and the loads run two slices (of this tile or the first of
+// the wave's next tile) ahead of the MFMAs.  Two forms: gemm_mfma below for single
+// products in LDS or memory, gemm_tiles_buf for the walkers' products.
 // ---------------------------------------------------------------------------
-
-// Run of NV operand values at k = kb..kb+NV-1 of one row of op(X), inside the
-// matrix: KC -- stored along k (p[kk]), else p[ld kk].  vec: KC with p + kb
-// 16-byte aligned.
-template <bool KC, int NV>
-__device__ __forceinline__ void load_run(const float *p, int ld, int kb, bool vec, float (&v)[NV]) {
-    if (KC && vec) {
-        const float4 *q = (const float4 *)(p + kb);
-#pragma unroll
-        for (int j = 0; j < NV / 4; ++j) {
-            const float4 x = q[j];
-            v[4 * j] = x.x;
-            v[4 * j + 1] = x.y;
-            v[4 * j + 2] = x.z;
-            v[4 * j + 3] = x.w;
-        }
-    } else {
-#pragma unroll
-        for (int u = 0; u < NV; ++u) v[u] = KC ? p[kb + u] : p[(size_t)ld * (kb + u)];
-    }
-}
-
-// The same run with zeros at k >= kmax.
-template <bool KC, int NV>
-__device__ __forceinline__ void load_run_pred(const float *p, int ld, int kb, int kmax, float (&v)[NV]) {
-#pragma unroll
-    for (int u = 0; u < NV; ++u) {
-        const int kk = kb + u;
-        v[u] = kk < kmax ? (KC ? p[kk] : p[(size_t)ld * kk]) : 0.f;
-    }
-}
 
 // 16-byte loads along k need 16-byte aligned bases, leading dimension and batch stride
 __device__ __forceinline__ bool aligned16(const float *X0, const float *X1, int ld, long s) {
@@ -215,23 +181,6 @@ struct TileGeom {
     static constexpr int KL = TS == 32 ? 8 : 4;  // k values per lane and slice
     static constexpr int NACC = TS == 32 ? 16 : 4;
 };
-
-// Lane operand pointers of tile tb (of all nb products) and term seg: the
-// lane's row of op(A) and its NW columns of op(B), clamped into the matrices.
-template <bool TA, bool TB, int TS, int NW>
-__device__ __forceinline__ void tile_ptrs(int tb, int seg, int m, int n, int tm, int tn, const float *A0,
-                                          const float *A1, int lda, const float *B0, const float *B1, int ldb, long sA,
-                                          long sB, int r, const float *&pa, const float *(&pb)[NW]) {
-    const int bt = tb / (tm * tn), t = tb - bt * (tm * tn);
-    const int ar = min((t % tm) * TS + r, m - 1);
-    const float *A = (seg ? A1 : A0) + (size_t)bt * sA, *B = (seg ? B1 : B0) + (size_t)bt * sB;
-    pa = TA ? A + (size_t)lda * ar : A + ar;
-#pragma unroll
-    for (int q = 0; q < NW; ++q) {
-        const int bc = min((t / tm) * TS * NW + TS * q + r, n - 1);
-        pb[q] = TB ? B + bc : B + (size_t)ldb * bc;
-    }
-}
 
 template <int TS, int NW>
 __device__ __forceinline__ void tile_store(float *C0, int ldc, long sC, int tb, int m, int n, int tm, int tn, int r,
@@ -301,70 +250,6 @@ __device__ __forceinline__ void buf_ld4(__amdgpu_buffer_rsrc_t r, int voff, floa
     v[3] = x.w;
 }
 
-// k a positive multiple of 16: every wave runs one pipelined chain over the
-// (tile, term, slice) items of its tiles.  The operands of the item two ahead
-// are loaded unconditionally (past the end the last item reloads itself) with
-// a fixed instruction sequence, so the wait for an item's operands covers only
-// its own loads.
-// VEC: the operands stored along k are 16-byte aligned (float4 loads).
-template <bool TA, bool TB, int TS, int NW, bool VEC>
-__device__ __forceinline__ void gemm_tiles_full(int m, int n, int k, const float *A0, const float *A1, int lda,
-                                             const float *B0, const float *B1, int ldb, float *C0, int ldc, bool acc,
-                                             int nseg, int nb, long sA, long sB, long sC) {
-    constexpr int KL = TileGeom<TS>::KL, NACC = TileGeom<TS>::NACC;
-    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r = lane % TS, h = lane / TS;
-    const int tm = (m + TS - 1) / TS, tn = (n + TS * NW - 1) / (TS * NW), ntile = nb * tm * tn;
-    if (w >= ntile) return;
-    const int ntw = (ntile - w + MQE_WAVES - 1) / MQE_WAVES;  // tiles of this wave
-    const int nsk = k >> 4, nsl = nseg * nsk, nit = ntw * nsl;
-    auto load = [&](int i, float (&a)[KL], float (&b)[NW][KL]) {
-        const int j = i / nsl, rem = i - j * nsl, seg = rem / nsk, sl = rem - seg * nsk;
-        const float *pa, *pb[NW];
-        tile_ptrs<TA, TB, TS, NW>(w + MQE_WAVES * j, seg, m, n, tm, tn, A0, A1, lda, B0, B1, ldb, sA, sB, r, pa, pb);
-        const int kb = 16 * sl + KL * h;
-        load_run<TA, KL>(pa, lda, kb, VEC, a);
-#pragma unroll
-        for (int q = 0; q < NW; ++q) load_run<!TB, KL>(pb[q], ldb, kb, VEC, b[q]);
-    };
-    // three operand sets in rotation (the loop is unrolled by three, so no
-    // register copies wait on loads in flight): the loads run two items ahead
-    // of the MFMAs
-    float a0[KL], b0[NW][KL], a1[KL], b1[NW][KL], a2[KL], b2[NW][KL], c[NW][NACC];
-#pragma unroll
-    for (int q = 0; q < NW; ++q)
-#pragma unroll
-        for (int e = 0; e < NACC; ++e) c[q][e] = 0.f;
-    auto step = [&](int i, const float (&a)[KL], const float (&b)[NW][KL]) {
-#pragma unroll
-        for (int u = 0; u < KL; ++u)
-#pragma unroll
-            for (int q = 0; q < NW; ++q) mfma_step<TS>(a[u], b[q][u], c[q]);
-        if ((i + 1) % nsl == 0) {  // the tile is complete
-            tile_store<TS, NW>(C0, ldc, sC, w + MQE_WAVES * (i / nsl), m, n, tm, tn, r, h, acc, c);
-#pragma unroll
-            for (int q = 0; q < NW; ++q)
-#pragma unroll
-                for (int e = 0; e < NACC; ++e) c[q][e] = 0.f;
-        }
-    };
-    load(0, a0, b0);
-    load(min(1, nit - 1), a1, b1);
-    for (int i = 0; i < nit; i += 3) {
-        load(min(i + 2, nit - 1), a2, b2);
-        __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of the MFMAs
-        step(i, a0, b0);
-        if (i + 1 >= nit) break;
-        load(min(i + 3, nit - 1), a0, b0);
-        __builtin_amdgcn_sched_barrier(0);
-        step(i + 1, a1, b1);
-        if (i + 2 >= nit) break;
-        load(min(i + 4, nit - 1), a1, b1);
-        __builtin_amdgcn_sched_barrier(0);
-        step(i + 2, a2, b2);
-    }
-}
-
 // Run of NV operand values of a slice through a buffer resource: voff the lane's
 // byte offset, soff the slice's, step the bytes per k (stored across k), left the
 // values of the lane's run inside the matrix (TAIL: the others read 0).
@@ -391,10 +276,13 @@ __device__ __forceinline__ void load_run_buf(__amdgpu_buffer_rsrc_t r, int voff,
     }
 }
 
-// The same chain for operands in global memory with uniform shapes (bonds above
-// 64): a cursor in scalar registers steps through the (tile, term, slice) items,
-// each load is one instruction (scalar slice offset, the lane's offset of the
-// tile), and a last partial slice reads zeros past k.  One wave per SIMD has to
+// C(m x n) = sum_{s < nseg} op(A_s) op(B_s) (nseg = 1 or 2 terms of one shape and
+// leading dimensions), for nb products at once (A_s + b sA and so on; their tiles are
+// shared among the four waves), operands in global memory, uniform shapes (bonds above
+// 64).  acc: C += instead of C =.  A cursor in scalar registers steps through the
+// (tile, term, slice) items, each load is one instruction (scalar slice offset, the
+// lane's offset of the tile) issued two items ahead of its MFMAs, and a last partial
+// slice reads zeros past k.  One wave per SIMD has to
 // issue everything between its MFMAs itself: with the operand addresses formed
 // from the item's number per load (divisions, 64-bit vector arithmetic) a step of
 // 256 walkers of the 6x6 snake at D = 128 took 151 ms, with the cursor 141 ms in
@@ -499,60 +387,103 @@ __device__ __forceinline__ void gemm_tiles_buf(int m, int n, int k, const float 
     }
 }
 
-// Any k: per tile and slice, predicated loads (zeros at k >= k), no pipelining.
-template <bool TA, bool TB, int TS, int NW>
-__device__ __forceinline__ void gemm_tiles_pred(int m, int n, int k, const float *A0, const float *A1, int lda,
-                                             const float *B0, const float *B1, int ldb, float *C0, int ldc, bool acc,
-                                             int nseg, int nb, long sA, long sB, long sC) {
-    constexpr int KL = TileGeom<TS>::KL, NACC = TileGeom<TS>::NACC;
+// C = op(A) op(B), operands in LDS or memory (the proposal network's layers), in
+// 32 x 32 tiles.  k a multiple of 16 and 16-byte aligned operands along k: one
+// pipelined chain over the (tile, slice) items of a wave, the operands of the item two
+// ahead loaded unconditionally (past the end the last item reloads itself) with a fixed
+// instruction sequence, so the wait for an item's operands covers only its own loads.
+// Else: per tile and slice, zeros at k and beyond, no pipelining.
+template <bool TA, bool TB>
+__device__ __forceinline__ void gemm_mfma(int m, int n, int k, const float *A, int lda, const float *B, int ldb,
+                                          float *C, int ldc) {
+    constexpr int TS = 32, KL = TileGeom<TS>::KL, NACC = TileGeom<TS>::NACC;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane % TS, h = lane / TS;
-    const int tm = (m + TS - 1) / TS, tn = (n + TS * NW - 1) / (TS * NW), ntile = nb * tm * tn;
-    for (int tb = w; tb < ntile; tb += MQE_WAVES) {
-        float c[NW][NACC];
+    const int tm = (m + TS - 1) / TS, tn = (n + TS - 1) / TS, ntile = tm * tn;
+    if (w >= ntile) return;
+    // a lane's row of op(A) and column of op(B) in tile t, clamped into the matrices
+    auto row = [&](int t) {
+        const int ar = min((t % tm) * TS + r, m - 1);
+        return TA ? A + (size_t)lda * ar : A + ar;
+    };
+    auto col = [&](int t) {
+        const int bc = min((t / tm) * TS + r, n - 1);
+        return TB ? B + bc : B + (size_t)ldb * bc;
+    };
+    float c[1][NACC];
 #pragma unroll
-        for (int q = 0; q < NW; ++q)
+    for (int e = 0; e < NACC; ++e) c[0][e] = 0.f;
+    if (k >= 16 && (k & 15) == 0 && (!TA || aligned16(A, A, lda, 0)) && (TB || aligned16(B, B, ldb, 0))) {
+        // KC: stored along k
+        auto run = [&](auto KC, const float *p, int ld, int kb, float (&v)[KL]) {
+            if constexpr (decltype(KC)::value) {
+                const float4 *q = (const float4 *)(p + kb);
 #pragma unroll
-            for (int e = 0; e < NACC; ++e) c[q][e] = 0.f;
-        for (int seg = 0; seg < nseg; ++seg) {
-            const float *pa, *pb[NW];
-            tile_ptrs<TA, TB, TS, NW>(tb, seg, m, n, tm, tn, A0, A1, lda, B0, B1, ldb, sA, sB, r, pa, pb);
-            for (int k0 = 0; k0 < k; k0 += 16) {
-                float a[KL], b[NW][KL];
-                load_run_pred<TA, KL>(pa, lda, k0 + KL * h, k, a);
+                for (int j = 0; j < KL / 4; ++j) {
+                    const float4 x = q[j];
+                    v[4 * j] = x.x;
+                    v[4 * j + 1] = x.y;
+                    v[4 * j + 2] = x.z;
+                    v[4 * j + 3] = x.w;
+                }
+            } else {
 #pragma unroll
-                for (int q = 0; q < NW; ++q) load_run_pred<!TB, KL>(pb[q], ldb, k0 + KL * h, k, b[q]);
-#pragma unroll
-                for (int u = 0; u < KL; ++u)
-#pragma unroll
-                    for (int q = 0; q < NW; ++q) mfma_step<TS>(a[u], b[q][u], c[q]);
+                for (int u = 0; u < KL; ++u) v[u] = p[(size_t)ld * (kb + u)];
             }
+        };
+        const int ntw = (ntile - w + MQE_WAVES - 1) / MQE_WAVES;  // tiles of this wave
+        const int nsl = k >> 4, nit = ntw * nsl;
+        auto load = [&](int i, float (&a)[KL], float (&b)[KL]) {
+            const int j = i / nsl, kb = 16 * (i - j * nsl) + KL * h, t = w + MQE_WAVES * j;
+            run(std::integral_constant<bool, TA>(), row(t), lda, kb, a);
+            run(std::integral_constant<bool, !TB>(), col(t), ldb, kb, b);
+        };
+        // three operand sets in rotation (the loop is unrolled by three, so no
+        // register copies wait on loads in flight)
+        float a0[KL], b0[KL], a1[KL], b1[KL], a2[KL], b2[KL];
+        auto step = [&](int i, const float (&a)[KL], const float (&b)[KL]) {
+#pragma unroll
+            for (int u = 0; u < KL; ++u) mfma_step<TS>(a[u], b[u], c[0]);
+            if ((i + 1) % nsl == 0) {  // the tile is complete
+                tile_store<TS, 1>(C, ldc, 0, w + MQE_WAVES * (i / nsl), m, n, tm, tn, r, h, false, c);
+#pragma unroll
+                for (int e = 0; e < NACC; ++e) c[0][e] = 0.f;
+            }
+        };
+        load(0, a0, b0);
+        load(min(1, nit - 1), a1, b1);
+        for (int i = 0; i < nit; i += 3) {
+            load(min(i + 2, nit - 1), a2, b2);
+            __builtin_amdgcn_sched_barrier(0);  // keep the loads ahead of the MFMAs
+            step(i, a0, b0);
+            if (i + 1 >= nit) break;
+            load(min(i + 3, nit - 1), a0, b0);
+            __builtin_amdgcn_sched_barrier(0);
+            step(i + 1, a1, b1);
+            if (i + 2 >= nit) break;
+            load(min(i + 4, nit - 1), a1, b1);
+            __builtin_amdgcn_sched_barrier(0);
+            step(i + 2, a2, b2);
         }
-        tile_store<TS, NW>(C0, ldc, sC, tb, m, n, tm, tn, r, h, acc, c);
+        return;
     }
-}
-
-template <bool TA, bool TB, int TS, int NW>
-__device__ __forceinline__ void gemm_tiles(int m, int n, int k, const float *A0, const float *A1, int lda,
-                                           const float *B0, const float *B1, int ldb, float *C0, int ldc, bool acc,
-                                           int nseg, int nb, long sA, long sB, long sC) {
-    // the pipelined path needs whole slices and 16-byte aligned operands stored
-    // along k (bond dimensions that are multiples of 16 give both)
-    const bool vec = (!TA || aligned16(A0, nseg > 1 ? A1 : A0, lda, sA)) &&
-                     (TB || aligned16(B0, nseg > 1 ? B1 : B0, ldb, sB));
-    if (k >= 16 && (k & 15) == 0 && vec) {
-        gemm_tiles_full<TA, TB, TS, NW, true>(m, n, k, A0, A1, lda, B0, B1, ldb, C0, ldc, acc, nseg, nb, sA, sB, sC);
-    } else {
-        gemm_tiles_pred<TA, TB, TS, NW>(m, n, k, A0, A1, lda, B0, B1, ldb, C0, ldc, acc, nseg, nb, sA, sB, sC);
+    for (int t = w; t < ntile; t += MQE_WAVES) {
+        const float *pa = row(t), *pb = col(t);
+#pragma unroll
+        for (int e = 0; e < NACC; ++e) c[0][e] = 0.f;
+        for (int k0 = 0; k0 < k; k0 += 16) {
+            float a[KL], b[KL];
+#pragma unroll
+            for (int u = 0; u < KL; ++u) {
+                const int kk = k0 + KL * h + u;
+                a[u] = kk < k ? (TA ? pa[kk] : pa[(size_t)lda * kk]) : 0.f;
+                b[u] = kk < k ? (TB ? pb[(size_t)ldb * kk] : pb[kk]) : 0.f;
+            }
+#pragma unroll
+            for (int u = 0; u < KL; ++u) mfma_step<TS>(a[u], b[u], c[0]);
+        }
+        tile_store<TS, 1>(C, ldc, 0, t, m, n, tm, tn, r, h, false, c);
     }
-}
-
-// Single products with operands in LDS or memory (the proposal network's layers).
-template <bool TA, bool TB>
-__device__ __forceinline__ void gemm_mfma(int m, int n, int k, const float *A0, int lda, const float *B0, int ldb,
-                                          float *C0, int ldc, bool acc, int nb = 1, long sA = 0, long sB = 0,
-                                          long sC = 0) {
-    gemm_tiles<TA, TB, 32, 1>(m, n, k, A0, A0, lda, B0, B0, ldb, C0, ldc, acc, 1, nb, sA, sB, sC);
 }
 
 // Output tile shapes of the FP32 matrix-core products (chosen per walker bond

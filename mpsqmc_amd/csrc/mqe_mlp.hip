@@ -106,15 +106,15 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
         xs[e] = r < 0 ? 0.f : (X[r * nin + f] - xm[f]) / xsd[f];
     }
     __syncthreads();
-    gemm_mfma<false, false>(H, TS, nin, W1, H, xs, nin, h1, lh, false);
+    gemm_mfma<false, false>(H, TS, nin, W1, H, xs, nin, h1, lh);
     __syncthreads();
     bias_act(h1, H, lh, b1, true);
     __syncthreads();
-    gemm_mfma<false, false>(H, TS, H, W2, H, h1, lh, h2, lh, false);
+    gemm_mfma<false, false>(H, TS, H, W2, H, h1, lh, h2, lh);
     __syncthreads();
     bias_act(h2, H, lh, b2, true);
     __syncthreads();
-    gemm_mfma<false, false>(nout, TS, H, W3, nout, h2, lh, o, lo, false);
+    gemm_mfma<false, false>(nout, TS, H, W3, nout, h2, lh, o, lo);
     __syncthreads();
     bias_act(o, nout, lo, b3, false);
     __syncthreads();
@@ -147,8 +147,8 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
         float *gW1 = G, *gb1 = G + off_b1(nin, H), *gW2 = G + off_W2(nin, H), *gb2 = G + off_b2(nin, H),
               *gW3 = G + off_W3(nin, H), *gb3 = G + off_b3(nin, H, nout);
         // layer 3: gW3 = dO h2^T, gb3 = rows of dO, dh2 = W3^T dO masked by h2 > 0
-        gemm_mfma<false, true>(nout, H, TS, o, lo, h2, lh, gW3, nout, false);
-        gemm_mfma<true, false>(H, TS, nout, W3, nout, o, lo, dh2, lh, false);
+        gemm_mfma<false, true>(nout, H, TS, o, lo, h2, lh, gW3, nout);
+        gemm_mfma<true, false>(H, TS, nout, W3, nout, o, lo, dh2, lh);
         for (int q = threadIdx.x; q < nout; q += MQE_NT) {
             float s = 0.f;
             for (int j = 0; j < TS; ++j) s += o[q + lo * j];
@@ -159,8 +159,8 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
             if (!(h2[e] > 0.f)) dh2[e] = 0.f;
         __syncthreads();
         // layer 2: gW2 = dh2 h1^T, gb2, dh1 = W2^T dh2 (into h2) masked by h1 > 0
-        gemm_mfma<false, true>(H, H, TS, dh2, lh, h1, lh, gW2, H, false);
-        gemm_mfma<true, false>(H, TS, H, W2, H, dh2, lh, h2, lh, false);
+        gemm_mfma<false, true>(H, H, TS, dh2, lh, h1, lh, gW2, H);
+        gemm_mfma<true, false>(H, TS, H, W2, H, dh2, lh, h2, lh);
         for (int q = threadIdx.x; q < H; q += MQE_NT) {
             float s = 0.f;
             for (int j = 0; j < TS; ++j) s += dh2[q + lh * j];
@@ -171,7 +171,7 @@ __global__ __launch_bounds__(MQE_NT) void tile_kernel(Net net, const float *X, c
             if (!(h1[e] > 0.f)) h2[e] = 0.f;
         __syncthreads();
         // layer 1: gW1 = dh1 xs^T, gb1
-        gemm_mfma<false, true>(H, nin, TS, h2, lh, xs, nin, gW1, H, false);
+        gemm_mfma<false, true>(H, nin, TS, h2, lh, xs, nin, gW1, H);
         for (int q = threadIdx.x; q < H; q += MQE_NT) {
             float s = 0.f;
             for (int j = 0; j < TS; ++j) s += h2[q + lh * j];
