@@ -402,7 +402,7 @@ __device__ int rscan_excl(int v, int *out_excl, int *sh) {
 struct Book {
     int *n;
     int *order, *order2;
-    double *w, *O, *eh, *EL;
+    double *w, *eh, *EL;
     double *sums;     // [0] sum w  [1] scaling  [2] E_T  [3] E_P  [4] Omega  [5] N
     double *trace;    // 6 doubles per step
     int *ncopy, *newpos, *used, *freelist, *copy_src, *copy_dst, *n_extra, *n_new, *n_used;
@@ -887,7 +887,6 @@ static Book make_book(mqe_engine *e) {
     B.order = e->d_order;
     B.order2 = e->d_order2;
     B.w = e->d_w;
-    B.O = e->d_O;
     B.eh = e->d_eh;
     B.EL = e->d_EL;
     B.sums = e->d_sums;
@@ -1346,11 +1345,6 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
     CK(hipMalloc((void **)&e->d_idx, sizeof(int) * std::max(nC, 1) * (size_t)cap));
     e->scratch_bytes = e->fp32 ? scratch_bytes_for<float>(e->Dt, e->Dw, n_grid)
                                : scratch_bytes_for<double>(e->Dt, e->Dw, n_grid);
-    {
-        // the overlap kernel needs 3 * Dmax^2 elements of T in the same scratch
-        long need = 3L * 4096 * 4096;  // upper bound used only if larger than the step scratch
-        (void)need;
-    }
     CK(hipMalloc((void **)&e->d_scratch, (size_t)e->scratch_bytes * cap));
     CK(hipMalloc((void **)&e->d_status, sizeof(int)));
     CK(hipMemset(e->d_status, 0, sizeof(int)));

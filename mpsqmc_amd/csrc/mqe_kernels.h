@@ -94,7 +94,7 @@ struct Pool {
 // Scratch layout of one workgroup (sizes in elements).
 struct ScratchLayout {
     long Y, Y4, G, GcA, GcB, W, V, TMP, LM, t_total;  // T region
-    long AQ, RQ, TAU, PARTS, DOTS, PDF, CUM, d_total;     // double region
+    long AQ, RQ, TAU, PDF, CUM, d_total;              // double region
 };
 
 __host__ __device__ inline ScratchLayout scratch_layout(int Dt, int Dw, int Ng) {
@@ -116,8 +116,6 @@ __host__ __device__ inline ScratchLayout scratch_layout(int Dt, int Dw, int Ng) 
     s.AQ = o; o += 2L * Dw * Dw > panels ? 2L * Dw * Dw : panels;
     s.RQ = o; o += (long)Dw * Dw;
     s.TAU = o; o += Dw;
-    s.PARTS = o; o += MQE_NT;
-    s.DOTS = o; o += (Dw > MQE_NT ? Dw : MQE_NT);
     s.PDF = o; o += Ng;
     s.CUM = o; o += Ng;
     s.d_total = o;
