@@ -48,13 +48,35 @@ __device__ __forceinline__ double readlane_d_(double v, int l) {
     return __hiloint2double(hi, lo);
 }
 
-// sum over aligned groups of 8 lanes (xor 1, xor 2 inside quads, then the
-// mirrored half-row), every lane of the group receives the sum
-__device__ __forceinline__ double group8_sum(double v) {
-    v += dpp_d<0xB1>(v);   // quad_perm [1,0,3,2]
-    v += dpp_d<0x4E>(v);   // quad_perm [2,3,0,1]
-    v += dpp_d<0x141>(v);  // row_half_mirror
+// sum over aligned groups of G = 4, 8 or 16 lanes; every lane receives it
+template <int G>
+__device__ __forceinline__ double lanes_sum(double v) {
+    v += dpp_d<0xB1>(v);                            // quad_perm [1,0,3,2]
+    v += dpp_d<0x4E>(v);                            // quad_perm [2,3,0,1]
+    if constexpr (G >= 8) v += dpp_d<0x141>(v);   // row_half_mirror
+    if constexpr (G >= 16) v += dpp_d<0x140>(v);  // row_mirror
     return v;
+}
+
+// (x, y) -> x + y of the partner half: for lanes 0-31 x(l) + x(l + 32), for
+// lanes 32-63 y(l - 32) + y(l), with one v_permlane32_swap per dword
+__device__ __forceinline__ double halves_sum(double x, double y) {
+    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(x), (unsigned)__double2loint(y),
+                                                     false, false);
+    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y),
+                                                     false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+}
+
+// (x, y) -> for 16-lane rows 0 and 2 x(l) + x(l + 16), for rows 1 and 3
+// y(l - 16) + y(l), with one v_permlane16_swap per dword (it returns rows
+// (x0, y0, x2, y2) and (x1, y1, x3, y3); checked on gfx950)
+__device__ __forceinline__ double rows_sum(double x, double y) {
+    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(x), (unsigned)__double2loint(y),
+                                                     false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y),
+                                                     false, false);
+    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
 }
 
 // DPP move of a double with a row mask; lanes of disabled rows receive 0
@@ -1016,16 +1038,6 @@ __device__ __forceinline__ void householder_qr(const QRCols &col, int n, double 
         }
     }
     __syncthreads();
-}
-
-// sum over aligned groups of G = 4, 8 or 16 lanes; every lane receives it
-template <int G>
-__device__ __forceinline__ double lanes_sum(double v) {
-    v += dpp_d<0xB1>(v);                            // quad_perm [1,0,3,2]
-    v += dpp_d<0x4E>(v);                            // quad_perm [2,3,0,1]
-    if constexpr (G >= 8) v += dpp_d<0x141>(v);   // row_half_mirror
-    if constexpr (G >= 16) v += dpp_d<0x140>(v);  // row_mirror
-    return v;
 }
 
 // 1 / sqrt(x) and 1 / x of a positive normal x to within rounding: the hardware's

@@ -60,23 +60,6 @@ __device__ __forceinline__ float dot4(v4 a, v4 b) { return a[0] * b[0] + a[1] * 
 
 __device__ __forceinline__ v4 unit_tile(Lane l) { return v4{l.j == 0 && l.g == 0 ? 1.f : 0.f, 0.f, 0.f, 0.f}; }
 
-// (x, y) -> lanes 0-31: x(l) + x(l + 32), lanes 32-63: y(l - 32) + y(l)
-__device__ __forceinline__ double halves_sum(double x, double y) {
-    const auto lo = __builtin_amdgcn_permlane32_swap((unsigned)__double2loint(x), (unsigned)__double2loint(y), false,
-                                                     false);
-    const auto hi = __builtin_amdgcn_permlane32_swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y), false,
-                                                     false);
-    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-}
-// the same between neighbouring 16-lane rows: even rows x, odd rows y
-__device__ __forceinline__ double rows_sum(double x, double y) {
-    const auto lo = __builtin_amdgcn_permlane16_swap((unsigned)__double2loint(x), (unsigned)__double2loint(y), false,
-                                                     false);
-    const auto hi = __builtin_amdgcn_permlane16_swap((unsigned)__double2hiint(x), (unsigned)__double2hiint(y), false,
-                                                     false);
-    return __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
-}
-
 // sixteen wave-wide sums by a reduce-scatter: lane l receives the sum of s[l / 4]
 __device__ __forceinline__ double reduce16(const double (&s)[16]) {
     const int lane = threadIdx.x & 63;
