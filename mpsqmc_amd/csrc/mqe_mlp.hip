@@ -40,10 +40,12 @@ namespace mlp {
 // 16,384 rows 88 -> 79 us; with the padded blocks below 80 and 71 us.
 constexpr int TS = 32;
 constexpr int MAX_IN = 32, MAX_H = 128, MAX_OUT = 32;
-// Gradient slots, and so the tiles of one training launch: twice as many as
-// workgroups that fit the chip (two a CU at H = 128).  90 MB at H = 128 whatever the
-// number of rows; a slot for every tile took 2.7 KB a row.
-constexpr long SLOTS = 1024;
+// Gradient slots, and so the tiles of one training launch: four times as many as
+// workgroups that fit the chip (two a CU at H = 128), so that the last, partly filled
+// round of a launch and the launch itself weigh little (65,536 rows: 620 us a call in
+// one launch, 656 in two of 1024 tiles).  180 MB at H = 128 whatever the number of
+// rows; a slot for every tile took 2.7 KB a row.
+constexpr long SLOTS = 2048;
 
 struct Net {
     int nin, H, nout;

@@ -1,5 +1,5 @@
 """The network's gradient over many rows: its workspace does not grow with them beyond a
-bound (1024 tiles of 32 rows), and more rows take turns in it.  One tile, exactly the
+bound (2048 tiles of 32 rows), and more rows take turns in it.  One tile, exactly the
 bound, one row and seven times more (the last tile ragged) against the FP64
 restatement at the gradient's bar, 1e-4 of its largest element; the step of an optimiser
 batch above the bound against the first step of Adam, lr sign(g)."""
@@ -21,7 +21,7 @@ def _free_bytes():
     return free.value
 
 
-@pytest.mark.parametrize("n", [31, 32768, 32769, 262143])
+@pytest.mark.parametrize("n", [31, 65536, 65537, 262143])
 def test_gradient_of_many_rows(n):
     H = 128
     net = MLP(NFEAT, H, NLABEL, seed=3)
@@ -34,8 +34,8 @@ def test_gradient_of_many_rows(n):
     before = _free_bytes()
     loss, g = net.loss_grad(X, Y)
     taken = before - _free_bytes()
-    # the rows (inputs, targets, outputs), 100 MB of gradients and the allocator's grain
-    assert taken <= 4 * n * (NFEAT + 2 * NLABEL) + (100 << 20) + (16 << 20)
+    # the rows (inputs, targets, outputs), 190 MB of gradients and the allocator's grain
+    assert taken <= 4 * n * (NFEAT + 2 * NLABEL) + (190 << 20) + (16 << 20)
     loss_o, g_o = omlp.loss_grad(p.astype(np.float64), X, Y, NFEAT, H, NLABEL)
     assert loss == pytest.approx(loss_o, rel=1e-5)
     assert np.max(np.abs(g - g_o)) <= 1e-4 * np.max(np.abs(g_o))
@@ -43,7 +43,7 @@ def test_gradient_of_many_rows(n):
 
 
 def test_adam_step_of_a_batch_above_the_bound():
-    n, H, lr = 40001, 32, 1e-3
+    n, H, lr = 70001, 32, 1e-3
     net = MLP(NFEAT, H, NLABEL, seed=4)
     p = net.params()
     rng = np.random.default_rng(5)
