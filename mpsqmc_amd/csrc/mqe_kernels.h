@@ -15,8 +15,8 @@ enum : int { F_PREP = 1, F_PROP = 2 };
 
 // Step control block in device memory.  The launches of a step read their
 // step-dependent values from here instead of taking them as arguments, so the
-// same launches can be captured once in a graph and replayed (a one-thread
-// kernel advances the block at the start of every captured step).
+// same launches can be captured once in a graph and replayed (the launch-list
+// kernel sets the block in an eager step and advances it in a captured one).
 struct Ctl {
     int step;         // device-RNG step word of the propagation; the energy's step number
     int pstep;        // device-RNG step word of population control

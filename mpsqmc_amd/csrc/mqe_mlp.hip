@@ -8,7 +8,7 @@
 // exact PDF value of the sampled point.  The reference has no such component.
 //
 // Kernels: one workgroup per tile of 32 samples.  The activations of a tile
-// stay in LDS (feature-major, ld = width); every layer product is a workgroup
+// stay in LDS (feature-major, padded leading dimension); every layer product is a workgroup
 // MFMA GEMM (v_mfma_f32_32x32x2f32) with the weights read from global memory
 // (80 KB at H = 128, L2-resident).  Training computes forward and backward of a
 // tile and writes the tile's gradient to its own slot; the Adam kernel sums the

@@ -18,7 +18,7 @@
 // The 32 x 32 kernel with its four waves spends eight times the matrix work on
 // such bonds (D <= 16 in 32 x 32 tiles) and two to four workgroup barriers per
 // coupling; one step with population control of 64 walkers of 10 sites at D = 8
-// takes 121 us (32 x 32: 260), of 1000 walkers of 50 sites 676 us (2003).
+// takes 119 us (32 x 32: 260), of 1000 walkers of 50 sites 690 us (2003).
 #ifndef MQE_TILE16_H
 #define MQE_TILE16_H
 

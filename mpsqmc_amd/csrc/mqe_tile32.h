@@ -12,8 +12,8 @@
 // One 256-thread workgroup (four wave64s) per walker.  Every 32x32x32 product
 // is one wave issuing 16 v_mfma_f32_32x32x2f32; the four waves work on
 // independent tiles between workgroup barriers.  QR (LQ) of the energy sweep is
-// FP64 Householder in LDS with one barrier per column; sampling, weights,
-// overlaps and energies are FP64.
+// FP64 Householder with its columns in registers, reflectors through LDS and one
+// barrier per column; sampling, weights, overlaps and energies are FP64.
 #ifndef MQE_TILE32_H
 #define MQE_TILE32_H
 
