@@ -35,6 +35,7 @@
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -785,7 +786,7 @@ struct mqe_engine {
     float *d_trialT = nullptr;  // chained general kernel: every T_k[s] transposed
     bool chained = false;       // the general kernel with chained products (bonds <= 64)
     hipStream_t stream = nullptr;
-    std::vector<float> stage;  // FP32: host staging of mqe_overlaps
+    std::unique_ptr<float[]> stage;  // FP32: host staging of mqe_overlaps (STAGE floats)
     unsigned long long pair_hash = 0;  // of the coupled pairs (key of the tile table)
     std::vector<int> tvd, wmax;
     std::vector<long> toff, woff, eoff, moff;
@@ -1111,7 +1112,7 @@ int overlaps_in_workspace(mqe_engine *e, const mqe_mps *other, double *out, char
         t += (long)other->vd[k] * other->vd[k + 1] * 2;
     }
     if (e->fp32) {
-        float *tmp = e->stage.data();
+        float *tmp = e->stage.get();
         for (long i0 = 0; i0 < pl.tot; i0 += STAGE) {
             const long m = std::min(STAGE, pl.tot - i0);
             for (long i = 0; i < m; ++i) tmp[i] = (float)other->data[i0 + i];
@@ -1172,7 +1173,7 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
     e->Ng = n_grid;
     e->gdim = grid_dim;
     e->fp32 = p->precision == MQE_PREC_FP32;
-    if (e->fp32) e->stage.resize(STAGE);
+    if (e->fp32) e->stage.reset(new float[STAGE]);
     e->tvd.assign(trial->vd, trial->vd + L + 1);
     e->Dt = *std::max_element(e->tvd.begin(), e->tvd.end());
     e->wmax.resize(L + 1);
