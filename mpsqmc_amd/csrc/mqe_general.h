@@ -834,7 +834,6 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
             // snake at D = 128, 256 walkers: 130 ms that way, 122 ms this way, of a
             // 15-site ring at D = 20, 200 walkers: 1317 and 1329 us)
             T *A = C.ts + C.sl.GcA, *B = C.ts + C.sl.GcB;
-            operator_channels(C, C.tv[k], C.wv[k], A, r_pending ? C.Rk(k) : nullptr);
             double ep = 0.0;
             int bond = k;
             for (int q = q0 + nq - 1; q >= q0; --q) {
@@ -844,6 +843,7 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
                 // barrier covers G)
                 if constexpr (CH) issue_G(C, i, C.Lk(i), C.ts + C.sl.G, 2 * tn, tn, (long)wn * 2 * tn, 0);
                 else compute_G(C, i, C.Lk(i));
+                if (bond == k) operator_channels(C, C.tv[k], C.wv[k], A, r_pending ? C.Rk(k) : nullptr);
                 for (; bond > i + 1; --bond) {
                     carry_left(C, bond - 1, A, B, 3);
                     T *t = A; A = B; B = t;
