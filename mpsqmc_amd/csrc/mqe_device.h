@@ -308,8 +308,8 @@ __device__ __forceinline__ void load_run_buf(__amdgpu_buffer_rsrc_t r, int voff,
 // issue everything between its MFMAs itself: with the operand addresses formed
 // from the item's number per load (divisions, 64-bit vector arithmetic) a step of
 // 256 walkers of the 6x6 snake at D = 128 took 151 ms, with the cursor 141 ms in
-// 32 x 32 and 130 ms in 32 x 64 tiles (with the energies' carries as they are now 137
-// and 121 ms).
+// 32 x 32 and 130 ms in 32 x 64 tiles (with the energies' carries as they are now 135
+// and 120 ms).
 // VEC: operands stored along k are 16-byte aligned and k is a multiple of 4.
 template <bool TA, bool TB, int TS, int NW, bool VEC>
 __device__ __forceinline__ void gemm_tiles_buf(int m, int n, int k, const float *A0, const float *A1, int lda,

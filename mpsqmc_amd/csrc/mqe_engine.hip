@@ -1405,7 +1405,7 @@ int mqe_create(const mqe_params *p, const mqe_mps *trial, int n_couplings, const
     S.ssp[0] = std::exp(0.5 * p->field * p->dtau * (-0.5));  // TrotterHeisenberg.cpp:86
     S.ssp[1] = std::exp(0.5 * p->field * p->dtau * (0.5));
     // above bonds of 64 two tiles per wave share an operand: a step of 256 walkers takes
-    // 121 ms instead of 137 for the 6x6 snake at D = 128, 10.8 instead of 11.6 for the
+    // 120 ms instead of 135 for the 6x6 snake at D = 128, 10.7 instead of 11.4 for the
     // 4x4 snake at D = 100
     for (int q = 0; q < 8; ++q) S.tiles[q] = q == 0 ? TILE_16 : q < 4 ? TILE_32 : TILE_WIDE;  // default table
     {
@@ -1724,7 +1724,7 @@ int mqe_kernel_path(mqe_engine *e) { return (e && e->tile32) ? 1 : 0; }
 // ---- tile-shape autotuner -----------------------------------------------------
 // Version of the products that the tables are tuned on.  A table is worth nothing on
 // other kernels (one tuned before the products above bonds of 64 were rewritten set
-// them back to 32 x 32 tiles: 137 instead of 121 ms a step of the 6x6 snake at
+// them back to 32 x 32 tiles: 135 instead of 120 ms a step of the 6x6 snake at
 // D = 128): raise it with every change of gemm_tiles_buf, the chained products, the
 // choice between them or the default table.
 constexpr int TILE_TABLE_VERSION = 2;

@@ -831,8 +831,8 @@ __device__ __forceinline__ double energy_sweep(const Ctx<T, CH> &C, double *O_ou
             // coupling meets the blocks G of its own first site and is summed, times J,
             // in FP64 (adding J S_i of the partners up in one set of FP32 channels
             // instead rounds every coupling to the largest of them; a step of the 6x6
-            // snake at D = 128, 256 walkers: 130 ms that way, 122 ms this way, of a
-            // 15-site ring at D = 20, 200 walkers: 1317 and 1329 us)
+            // snake at D = 128, 256 walkers: 130 ms that way, 120 ms this way, of a
+            // 15-site ring at D = 20, 200 walkers: 1317 and 1327 us)
             T *A = C.ts + C.sl.GcA, *B = C.ts + C.sl.GcB;
             double ep = 0.0;
             int bond = k;
